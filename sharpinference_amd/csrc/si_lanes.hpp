@@ -6,7 +6,7 @@
 namespace si {
 
 // The value that DPP control CTRL reads for this lane.  Every control used
-// by these kernels (quad_perm, row_half_mirror, row_mirror) reads a lane of
+// by these kernels (quad_perm, row_half_mirror, row_mirror, row_ror:8) reads a lane of
 // the reading lane's own 16-lane row, so no lane is out of range and
 // bound_ctrl changes no result; it lets the compiler fold the move into the
 // consumer as a DPP source operand (one v_add_f32_dpp / v_max_f32_dpp
@@ -14,7 +14,7 @@ namespace si {
 template <int CTRL>
 __device__ __forceinline__ int dpp_row(int v)
 {
-    static_assert(CTRL == 0xB1 || CTRL == 0x4E || CTRL == 0x141 || CTRL == 0x140,
+    static_assert(CTRL == 0xB1 || CTRL == 0x4E || CTRL == 0x141 || CTRL == 0x140 || CTRL == 0x128,
                   "controls whose source lane is always inside the row");
     return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true);
 }

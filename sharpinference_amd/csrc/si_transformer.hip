@@ -33,13 +33,6 @@ __device__ __forceinline__ float wave_sum_f(float v)
     return v;
 }
 
-__device__ __forceinline__ float wave_max_f(float v)
-{
-    for (int off = 32; off > 0; off >>= 1)
-        v = fmaxf(v, __shfl_xor(v, off));
-    return v;
-}
-
 // Sum over the workgroup (every thread gets it); `red` holds one float per wave.
 template <int THREADS>
 __device__ __forceinline__ float block_sum(float v, float* red)
@@ -52,21 +45,6 @@ __device__ __forceinline__ float block_sum(float v, float* red)
 #pragma unroll
     for (int w = 0; w < THREADS / 64; w++)
         t += red[w];
-    __syncthreads();
-    return t;
-}
-
-template <int THREADS>
-__device__ __forceinline__ float block_max(float v, float* red)
-{
-    v = wave_max_f(v);
-    if ((threadIdx.x & 63) == 0)
-        red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    float t = red[0];
-#pragma unroll
-    for (int w = 1; w < THREADS / 64; w++)
-        t = fmaxf(t, red[w]);
     __syncthreads();
     return t;
 }
@@ -149,143 +127,38 @@ __global__ __launch_bounds__(256) void rope_kv_write_kernel(RopeKvWriteArgs a, T
     }
 }
 
-// 8 consecutive cache values of one row as floats (one 16-byte fp16 load or
-// two 16-byte FP32 loads).
+// 8 consecutive floats (two 16-byte loads).
 __device__ __forceinline__ void load8(const float* p, float* f)
 {
     const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
     f[0] = a.x; f[1] = a.y; f[2] = a.z; f[3] = a.w;
     f[4] = b.x; f[5] = b.y; f[6] = b.z; f[7] = b.w;
 }
-__device__ __forceinline__ void load8(const __half* p, float* f)
-{
-    const uint4 r = *reinterpret_cast<const uint4*>(p);
-    const uint32_t w[4] = {r.x, r.y, r.z, r.w};
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        f[2 * k] = __half2float(__ushort_as_half(static_cast<unsigned short>(w[k] & 0xffffu)));
-        f[2 * k + 1] = __half2float(__ushort_as_half(static_cast<unsigned short>(w[k] >> 16)));
-    }
-}
-__device__ __forceinline__ float load1(const float* p) { return *p; }
-__device__ __forceinline__ float load1(const __half* p) { return __half2float(*p); }
 
 constexpr int GQA_THREADS = 256;
-constexpr int GQA_CHUNK = 64;      // cache rows per partial workgroup
+constexpr int GQA_CHUNK = 64;      // cache rows per partial of the workspace layout
 
-// One workgroup per (query head, 64-row chunk): scores of the chunk's rows
-// (head_size / 8 lanes per row, 8 channels each: coalesced row reads,
-// shuffle sums), the chunk's softmax maximum m and sum l, and its
-// unnormalised weighted sum of value rows o; partial (m, l, o[head]) goes
-// to the workspace.  Rows past the active range count as absent (weight 0);
-// a chunk wholly past it is never read by the merge.
-template <typename T, int HEAD>
-__global__ __launch_bounds__(GQA_THREADS) void gqa_partial_kernel(GqaArgs a, const T* __restrict__ kc,
-                                                                  const T* __restrict__ vc)
-{
-    __shared__ float scores[GQA_CHUNK];
-    __shared__ float red[GQA_THREADS / 64];
-    __shared__ float vpart[GQA_THREADS];
-    constexpr int LPT = HEAD / 8;                  // lanes per cache row
-    constexpr int ROWS = GQA_THREADS / LPT;        // rows per pass
-    constexpr int PASSES = GQA_CHUNK / ROWS;
-    const int head = blockIdx.x, chunk = blockIdx.y;
-    const int kvh = head / (a.query_heads / a.kv_heads);
-    const int active = min(max(*a.position, 0), a.context - 1);
-    const int t0 = chunk * GQA_CHUNK;
-    if (t0 > active)
-        return;                                    // whole workgroup: nothing to merge from this chunk
-    const int64_t row_stride = static_cast<int64_t>(a.kv_heads) * HEAD;
-    const float scale = 1.0f / sqrtf(static_cast<float>(HEAD));
-    const int part = threadIdx.x % LPT, sub = threadIdx.x / LPT;
-    float q[8];
-    load8(a.query + static_cast<int64_t>(head) * HEAD + 8 * part, q);
-    float k[PASSES][8];
-#pragma unroll
-    for (int i = 0; i < PASSES; i++) {
-        const int t = min(t0 + i * ROWS + sub, active);
-        load8(kc + static_cast<int64_t>(t) * row_stride + static_cast<int64_t>(kvh) * HEAD + 8 * part, k[i]);
-    }
-#pragma unroll
-    for (int i = 0; i < PASSES; i++) {
-        float s = 0.0f;
-#pragma unroll
-        for (int c = 0; c < 8; c++)
-            s = fmaf(q[c], k[i][c], s);
-#pragma unroll
-        for (int off = LPT / 2; off > 0; off >>= 1)
-            s += __shfl_xor(s, off);
-        const int r = i * ROWS + sub;
-        if (part == 0)
-            scores[r] = t0 + r <= active ? s * scale : -INFINITY;
-    }
-    __syncthreads();
-    float m = -INFINITY;
-    if (threadIdx.x < GQA_CHUNK)
-        m = scores[threadIdx.x];
-    m = block_max<GQA_THREADS>(m, red);            // finite: row t0 is active
-    float p = 0.0f;
-    if (threadIdx.x < GQA_CHUNK) {
-        p = expf(scores[threadIdx.x] - m);         // exp(-inf) = 0 for absent rows
-        scores[threadIdx.x] = p;
-    }
-    const float l = block_sum<GQA_THREADS>(p, red);   // its barriers also publish the weights
-    const int rows = min(GQA_CHUNK, active - t0 + 1);
-    float* dst = a.workspace + (static_cast<int64_t>(head) * a.chunks + chunk) * (HEAD + 2);
-    for (int d0 = 0; d0 < HEAD; d0 += GQA_THREADS / 2) {
-        const int d = d0 + threadIdx.x % (GQA_THREADS / 2), h2 = threadIdx.x / (GQA_THREADS / 2);
-        float acc = 0.0f;
-        if (d < HEAD) {
-            const T* vrow = vc + static_cast<int64_t>(t0) * row_stride + static_cast<int64_t>(kvh) * HEAD + d;
-            for (int r = h2; r < rows; r += 2)
-                acc = fmaf(scores[r], load1(vrow + static_cast<int64_t>(r) * row_stride), acc);
-        }
-        vpart[threadIdx.x] = acc;
-        __syncthreads();
-        if (h2 == 0 && d < HEAD)
-            dst[2 + d] = acc + vpart[threadIdx.x + GQA_THREADS / 2];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        dst[0] = m;
-        dst[1] = l;
-    }
-}
-
-// One workgroup per query head: out = sum_c o_c e^(m_c - M) / sum_c l_c e^(m_c - M)
-// over the active chunks, M = max_c m_c.
-template <int HEAD>
-__global__ __launch_bounds__(HEAD) void gqa_merge_kernel(GqaArgs a)
-{
-    const int head = blockIdx.x, d = threadIdx.x;
-    const int active = min(max(*a.position, 0), a.context - 1);
-    const int n = active / GQA_CHUNK + 1;
-    const float* src = a.workspace + static_cast<int64_t>(head) * a.chunks * (HEAD + 2);
-    float M = -INFINITY;
-    for (int c = 0; c < n; c++)
-        M = fmaxf(M, src[static_cast<int64_t>(c) * (HEAD + 2)]);
-    float L = 0.0f, O = 0.0f;
-    for (int c = 0; c < n; c++) {
-        const float* pc = src + static_cast<int64_t>(c) * (HEAD + 2);
-        const float e = expf(pc[0] - M);
-        L = fmaf(pc[1], e, L);
-        O = fmaf(pc[2 + d], e, O);
-    }
-    a.output[static_cast<int64_t>(head) * HEAD + d] = O / L;
-}
-
-// head_size 128, group G <= 4: one workgroup = one KV head x 128 cache rows
-// (the decode step's register-resident form, without its rotary and
-// append: rope-kv-write has already rotated the query and written the row).
-// Thread (wave w, lane l) takes the 8-value slice l % 16 of rows
-// 32 w + l / 16 + 4 j (j < 8) for both the scores and the values, so the
-// softmax weights stay in its registers: each wave keeps its maximum and
-// sum, sums across its four rows with lane swaps, and the four waves merge
-// (with rescaling) through LDS at one barrier.  Rows past the active range
-// count as absent.  Partials (m, l, o) of each query head and chunk go to
-// the workspace at the 64-row layout's index (chunk < its chunk count).
-constexpr int GQA_FCHUNK = 128;
-
+// One workgroup = one KV head x CHUNK cache rows x up to G query heads of its
+// group (grid z: the group in parts of at most 4 heads), every intermediate
+// in registers (the decode step's form, without its rotary and append:
+// rope-kv-write has already rotated the query and written the row).
+// A cache row's HEAD values are SL = HEAD / 8 slices of 8; thread (wave w,
+// lane l) takes slice l % SL of rows w * CHUNK / 4 + l / SL + RPW j for both
+// the scores and the values, so the softmax weights stay in its registers.
+// Every K and V row of the chunk is requested at once; each wave keeps its
+// own maximum, and the waves' rows merge (with rescaling) through LDS at the
+// kernel's one barrier.  Rows past the active range count as absent.
+// Partials (m, l, o) of each query head and chunk go to the workspace at the
+// 64-row layout's index (chunk < its chunk count).
+//
+// Bound: the round trips position -> cache rows -> partials (two launches a
+// call), not the cache bytes.  FP32 caches, 32 heads of 64 over 4 KV heads,
+// 4000 of 4096 rows, eight calls in a plan: 392 us with the staged form this
+// replaces (scores and weights through LDS, one workgroup per query head,
+// so a group's cache rows were read once per query head, and a merge that
+// walked the chunks one by one on 32 workgroups of one wave: 17 + 31 us a
+// call), 8.5 us a call now; 8 heads-of-128 groups of 4, fp16, 16000 of 16384
+// rows: 59.4 -> 22.2 us; 512-row FP32 cache, 8 heads over 4: 7.7 -> 5.9 us.
 template <typename T>
 struct CacheSlice {   // 8 consecutive values of one cache row as loaded
     uint4 w[sizeof(T) == 2 ? 1 : 2];
@@ -316,23 +189,48 @@ __device__ __forceinline__ void unpack_slice(const CacheSlice<float>& r, float* 
     f[6] = __uint_as_float(r.w[1].z); f[7] = __uint_as_float(r.w[1].w);
 }
 
-template <typename T, int G>
+// Sum over the SL (8, 16 or 32) lanes that hold one cache row.
+template <int SL>
+__device__ __forceinline__ float slice_sum(float v)
+{
+    v = row_sum<SL < 16 ? SL : 16>(v);
+    if constexpr (SL == 32) {
+        const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float(b[0]) + __uint_as_float(b[1]);
+    }
+    return v;
+}
+
+// Maximum over the wave of values that are equal within a row's SL lanes.
+template <int SL>
+__device__ __forceinline__ float slices_max(float v)
+{
+    if constexpr (SL == 8)
+        v = fmaxf(v, dpp_row<0x128>(v));   // the other row of the 16 lanes
+    return rows_max(v);
+}
+
+template <typename T, int HEAD, int G, int CHUNK>
 __global__ __launch_bounds__(GQA_THREADS) void gqa_chunk_kernel(GqaArgs a, const T* __restrict__ kc,
                                                                 const T* __restrict__ vc)
 {
-    constexpr int HEAD = 128, PPL = GQA_FCHUNK / 16;   // rows per lane
+    constexpr int SL = HEAD / 8, RPW = 64 / SL;        // lanes per cache row, rows per wave and step
+    constexpr int WROWS = CHUNK / 4, PPL = WROWS / RPW;   // rows per wave, per lane
+    static_assert(PPL * RPW * 4 == CHUNK, "whole rows per lane");
     const int g = blockIdx.x, chunk = blockIdx.y;
-    const int start = chunk * GQA_FCHUNK;
+    const int group = a.query_heads / a.kv_heads;
+    const int h0 = static_cast<int>(blockIdx.z) * G;   // first head of this part of the group
+    const int start = chunk * CHUNK;
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int dg = lane & 15, row = lane >> 4;
+    const int dg = lane & (SL - 1), row = lane / SL;
     float q[G][8];
 #pragma unroll
-    for (int h = 0; h < G; h++)
-        load8(a.query + static_cast<int64_t>(g * G + h) * HEAD + 8 * dg, q[h]);
+    for (int h = 0; h < G; h++)   // a last part with fewer heads repeats the group's last one and drops it
+        load8(a.query + static_cast<int64_t>(g * group + min(h0 + h, group - 1)) * HEAD + 8 * dg, q[h]);
     const int active = min(max(*a.position, 0), a.context - 1);
     const bool valid = start <= active;
-    const int count = min(GQA_FCHUNK, active + 1 - start);
+    const int count = min(CHUNK, active + 1 - start);
     const int64_t row_stride = static_cast<int64_t>(a.kv_heads) * HEAD;
     const T* kb = kc + static_cast<int64_t>(g) * HEAD + 8 * dg;
     const T* vb = vc + static_cast<int64_t>(g) * HEAD + 8 * dg;
@@ -340,18 +238,18 @@ __global__ __launch_bounds__(GQA_THREADS) void gqa_chunk_kernel(GqaArgs a, const
     if (valid) {   // a chunk past the active rows loads nothing and stores nothing
 #pragma unroll
         for (int j = 0; j < PPL; j++) {
-            const int64_t r = min(start + wave * (GQA_FCHUNK / 4) + row + 4 * j, a.context - 1);
+            const int64_t r = min(start + wave * WROWS + row + RPW * j, a.context - 1);
             kr[j] = load_slice(kb + r * row_stride);
             vr[j] = load_slice(vb + r * row_stride);
         }
     }
-    // scores q.k / sqrt(128) (a 16-lane row holds one cache row), masked
-    // past the count; exponentials with the hardware exp2 (__expf)
+    // scores q.k / sqrt(HEAD), masked past the count; exponentials with the
+    // hardware exp2 (__expf)
     const float rscale = 1.0f / sqrtf(static_cast<float>(HEAD));
     float sc[G][PPL];
 #pragma unroll
     for (int j = 0; j < PPL; j++) {
-        const int p = wave * (GQA_FCHUNK / 4) + row + 4 * j;
+        const int p = wave * WROWS + row + RPW * j;
         float k8[8];
         unpack_slice(kr[j], k8);
 #pragma unroll
@@ -360,7 +258,7 @@ __global__ __launch_bounds__(GQA_THREADS) void gqa_chunk_kernel(GqaArgs a, const
 #pragma unroll
             for (int e = 0; e < 8; e++)
                 d = fmaf(q[h][e], k8[e], d);
-            d = row_sum<16>(d);
+            d = slice_sum<SL>(d);
             sc[h][j] = p < count ? d * rscale : -INFINITY;
         }
     }
@@ -371,7 +269,7 @@ __global__ __launch_bounds__(GQA_THREADS) void gqa_chunk_kernel(GqaArgs a, const
 #pragma unroll
         for (int j = 1; j < PPL; j++)
             mh = fmaxf(mh, sc[h][j]);
-        mh = rows_max(mh);
+        mh = slices_max<SL>(mh);
         m[h] = mh;
         float lh = 0.0f;
 #pragma unroll
@@ -387,7 +285,7 @@ __global__ __launch_bounds__(GQA_THREADS) void gqa_chunk_kernel(GqaArgs a, const
     }
 #pragma unroll
     for (int j = 0; j < PPL; j++) {
-        const int p = wave * (GQA_FCHUNK / 4) + row + 4 * j;
+        const int p = wave * WROWS + row + RPW * j;
         float v8[8];
         unpack_slice(vr[j], v8);
 #pragma unroll
@@ -399,42 +297,43 @@ __global__ __launch_bounds__(GQA_THREADS) void gqa_chunk_kernel(GqaArgs a, const
             for (int e = 0; e < 8; e++)
                 acc[h][e] = fmaf(sc[h][j], v8[e], acc[h][e]);
     }
-    __shared__ float red[4][G][HEAD];
-    __shared__ float wm[4][G], wl[4][G];
+    __shared__ float4 red4[4 * RPW][G][HEAD / 4];
+    __shared__ float wm[4][G], wl[4 * RPW][G];
 #pragma unroll
     for (int h = 0; h < G; h++) {
-        l[h] = rows_sum(l[h]);
-#pragma unroll
-        for (int e = 0; e < 8; e++)
-            acc[h][e] = rows_sum(acc[h][e]);
+        red4[wave * RPW + row][h][2 * dg] = make_float4(acc[h][0], acc[h][1], acc[h][2], acc[h][3]);
+        red4[wave * RPW + row][h][2 * dg + 1] = make_float4(acc[h][4], acc[h][5], acc[h][6], acc[h][7]);
     }
-    if (row == 0) {
+    if (dg == 0)
 #pragma unroll
-        for (int h = 0; h < G; h++)
-#pragma unroll
-            for (int e = 0; e < 8; e++)
-                red[wave][h][8 * dg + e] = acc[h][e];
-        if (dg == 0)
-#pragma unroll
-            for (int h = 0; h < G; h++) {
+        for (int h = 0; h < G; h++) {
+            wl[wave * RPW + row][h] = l[h];
+            if (row == 0)
                 wm[wave][h] = m[h];
-                wl[wave][h] = l[h];
-            }
-    }
+        }
     __syncthreads();
     if (!valid)
         return;
+    const float* red = reinterpret_cast<const float*>(red4);
     for (int i = t; i < G * HEAD; i += GQA_THREADS) {
         const int h = i / HEAD, d = i % HEAD;
+        if (h0 + h >= group)
+            break;
         const float M = fmaxf(fmaxf(wm[0][h], wm[1][h]), fmaxf(wm[2][h], wm[3][h]));   // finite: row start is active
         float o = 0.0f, lsum = 0.0f;
 #pragma unroll
         for (int w = 0; w < 4; w++) {
             const float f = wm[w][h] == -INFINITY ? 0.0f : __expf(wm[w][h] - M);   // a wave without active rows adds nothing
-            o = fmaf(red[w][h][d], f, o);
-            lsum = fmaf(wl[w][h], f, lsum);
+            float ow = 0.0f, lw = 0.0f;
+#pragma unroll
+            for (int r = 0; r < RPW; r++) {
+                ow += red[((w * RPW + r) * G + h) * HEAD + d];
+                lw += wl[w * RPW + r][h];
+            }
+            o = fmaf(ow, f, o);
+            lsum = fmaf(lw, f, lsum);
         }
-        float* dst = a.workspace + (static_cast<int64_t>(g * G + h) * a.chunks + chunk) * (HEAD + 2);
+        float* dst = a.workspace + (static_cast<int64_t>(g * group + h0 + h) * a.chunks + chunk) * (HEAD + 2);
         dst[2 + d] = o;
         if (d == 0) {
             dst[0] = M;
@@ -443,43 +342,123 @@ __global__ __launch_bounds__(GQA_THREADS) void gqa_chunk_kernel(GqaArgs a, const
     }
 }
 
-// The merge of CHUNK-row partials: one workgroup per query head, batches of
-// 8 chunks requested together, merged online (m, l, o rescaled per batch).
-template <int HEAD, int CHUNK>
-__global__ __launch_bounds__(HEAD) void gqa_merge_chunks_kernel(GqaArgs a)
+// The merge of CHUNK-row partials, one workgroup per query head:
+// out = sum_c o_c e^(m_c - M) / sum_c l_c e^(m_c - M) over the active
+// chunks, M = max_c m_c.  SLOTS groups of HEAD threads take the chunks in
+// turn, each a batch of BATCH chunks per round trip merged online (m, l, o
+// rescaled per batch), and merge through LDS: up to BATCH * SLOTS chunks
+// cost one round trip, the first batch's requested before the position is
+// known.
+template <int HEAD, int CHUNK, int SLOTS, int BATCH>
+__global__ __launch_bounds__(HEAD * SLOTS) void gqa_merge_kernel(GqaArgs a)
 {
-    const int head = blockIdx.x, d = threadIdx.x;
+    const int head = blockIdx.x, d = threadIdx.x % HEAD, slot = threadIdx.x / HEAD;
+    const float* src = a.workspace + static_cast<int64_t>(head) * a.chunks * (HEAD + 2);
+    const int all = (a.context + CHUNK - 1) / CHUNK;   // partials a full cache has
     const int active = min(max(*a.position, 0), a.context - 1);
     const int n = active / CHUNK + 1;
-    const float* src = a.workspace + static_cast<int64_t>(head) * a.chunks * (HEAD + 2);
     float m = -INFINITY, L = 0.0f, O = 0.0f;
-    for (int c0 = 0; c0 < n; c0 += 8) {
-        float mc[8], lc[8], oc[8];
+    int c0 = slot;
+    do {   // the first batch's loads (any partial of the workspace) need no position
+        float mc[BATCH], lc[BATCH], oc[BATCH];
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const float* pc = src + static_cast<int64_t>(min(c0 + u, n - 1)) * (HEAD + 2);
+        for (int u = 0; u < BATCH; u++) {
+            const float* pc = src + static_cast<int64_t>(min(c0 + u * SLOTS, all - 1)) * (HEAD + 2);
             mc[u] = pc[0];
             lc[u] = pc[1];
             oc[u] = pc[2 + d];
         }
         float bm = m;
 #pragma unroll
-        for (int u = 0; u < 8; u++)
-            if (c0 + u < n)
-                bm = fmaxf(bm, mc[u]);
-        const float r = __expf(m - bm);   // m = -inf before the first batch: r = 0
+        for (int u = 0; u < BATCH; u++)
+            bm = c0 + u * SLOTS < n ? fmaxf(bm, mc[u]) : bm;
+        const float r = m == -INFINITY ? 0.0f : __expf(m - bm);
         L *= r;
         O *= r;
 #pragma unroll
-        for (int u = 0; u < 8; u++)
-            if (c0 + u < n) {
-                const float e = __expf(mc[u] - bm);
-                L = fmaf(lc[u], e, L);
-                O = fmaf(oc[u], e, O);
-            }
+        for (int u = 0; u < BATCH; u++) {   // partials past the active chunks may hold anything
+            const bool in = c0 + u * SLOTS < n;
+            const float e = in ? __expf(mc[u] - bm) : 0.0f;
+            L = fmaf(in ? lc[u] : 0.0f, e, L);
+            O = fmaf(in ? oc[u] : 0.0f, e, O);
+        }
         m = bm;
+        c0 += BATCH * SLOTS;
+    } while (c0 < n);
+    __shared__ float sm[SLOTS], sl[SLOTS], so[SLOTS][HEAD];
+    so[slot][d] = O;
+    if (d == 0) {
+        sm[slot] = m;
+        sl[slot] = L;
     }
-    a.output[static_cast<int64_t>(head) * HEAD + d] = O / L;
+    __syncthreads();
+    if (slot != 0)
+        return;
+    float M = sm[0];
+#pragma unroll
+    for (int s = 1; s < SLOTS; s++)
+        M = fmaxf(M, sm[s]);
+    float lsum = 0.0f, o = 0.0f;
+#pragma unroll
+    for (int s = 0; s < SLOTS; s++) {
+        const float e = __expf(sm[s] - M);   // a slot without chunks: m = -inf, e = 0
+        lsum = fmaf(sl[s], e, lsum);
+        o = fmaf(so[s][d], e, o);
+    }
+    a.output[static_cast<int64_t>(head) * HEAD + d] = o / lsum;
+}
+
+template <typename T, int HEAD, int G, int CHUNK>
+hipError_t launch_gqa_form(const GqaArgs& a, int parts, hipStream_t s)
+{
+    const int chunks = (a.context + CHUNK - 1) / CHUNK;
+    const dim3 grid(static_cast<unsigned>(a.kv_heads), static_cast<unsigned>(chunks), static_cast<unsigned>(parts));
+    hipLaunchKernelGGL((gqa_chunk_kernel<T, HEAD, G, CHUNK>), grid, dim3(GQA_THREADS), 0, s, a,
+                       static_cast<const T*>(a.key_cache), static_cast<const T*>(a.value_cache));
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess)
+        return e;
+    // one round trip for every chunk count of the cache (two at 256-value
+    // heads past 64 chunks), with no more slots and loads than that takes
+    const dim3 heads(static_cast<unsigned>(a.query_heads));
+    if (chunks <= 8)
+        hipLaunchKernelGGL((gqa_merge_kernel<HEAD, CHUNK, 1, 8>), heads, dim3(HEAD), 0, s, a);
+    else if (chunks <= 32)
+        hipLaunchKernelGGL((gqa_merge_kernel<HEAD, CHUNK, 4, 8>), heads, dim3(HEAD * 4), 0, s, a);
+    else {
+        constexpr int SLOTS = HEAD == 256 ? 4 : 8;
+        hipLaunchKernelGGL((gqa_merge_kernel<HEAD, CHUNK, SLOTS, 16>), heads, dim3(HEAD * SLOTS), 0, s, a);
+    }
+    return hipGetLastError();
+}
+
+// CHUNK: 128 rows where the whole cache then still gives a workgroup per CU
+// (half the partials to merge), 64 otherwise (2000-row cache, 8 KV heads of
+// 128: 8.8 us against 10.0 with 128 rows; 1 KV head, 16384 rows of 128 in
+// FP32: 13.2 against 15.9 with 128 rows only from 512 workgroups); 256-value
+// heads keep 64 (a lane's rows of a 128-row chunk would not fit its
+// registers).
+template <typename T, int HEAD, int G>
+hipError_t launch_gqa_group(const GqaArgs& a, int parts, hipStream_t s)
+{
+    if constexpr (HEAD < 256) {
+        if (static_cast<int64_t>(a.kv_heads) * parts * ((a.context + 127) / 128) >= 256)
+            return launch_gqa_form<T, HEAD, G, 128>(a, parts, s);
+    }
+    return launch_gqa_form<T, HEAD, G, 64>(a, parts, s);
+}
+
+template <typename T, int HEAD>
+hipError_t launch_gqa_head(const GqaArgs& a, hipStream_t s)
+{
+    const int group = a.query_heads / a.kv_heads;
+    const int parts = (group + 3) / 4;
+    switch ((group + parts - 1) / parts) {   // heads per part, evenly
+    case 1: return launch_gqa_group<T, HEAD, 1>(a, parts, s);
+    case 2: return launch_gqa_group<T, HEAD, 2>(a, parts, s);
+    case 3: return launch_gqa_group<T, HEAD, 3>(a, parts, s);
+    default: return launch_gqa_group<T, HEAD, 4>(a, parts, s);
+    }
 }
 
 }  // namespace
@@ -524,52 +503,14 @@ int64_t gqa_workspace_floats(int query_heads, int head_size, int context)
 
 hipError_t launch_gqa(const GqaArgs& a, hipStream_t s)
 {
-    const dim3 grid(static_cast<unsigned>(a.query_heads), static_cast<unsigned>(a.chunks));
-    const dim3 heads(static_cast<unsigned>(a.query_heads));
-    const int group = a.kv_heads > 0 ? a.query_heads / a.kv_heads : 0;
-    if (a.head_size == 128 && group >= 1 && group <= 4 && group * a.kv_heads == a.query_heads) {
-        // the register-resident form over 128-row chunks
-        const dim3 fgrid(static_cast<unsigned>(a.kv_heads), static_cast<unsigned>((a.context + GQA_FCHUNK - 1) / GQA_FCHUNK));
-        switch (group * 2 + (a.cache_fp16 ? 1 : 0)) {
-#define SI_GQA_CHUNK(G, F, T)                                                                                     \
-    case G * 2 + F:                                                                                               \
-        hipLaunchKernelGGL((gqa_chunk_kernel<T, G>), fgrid, dim3(GQA_THREADS), 0, s, a,                          \
-                           static_cast<const T*>(a.key_cache), static_cast<const T*>(a.value_cache));            \
-        break;
-        SI_GQA_CHUNK(1, 0, float)
-        SI_GQA_CHUNK(2, 0, float)
-        SI_GQA_CHUNK(3, 0, float)
-        SI_GQA_CHUNK(4, 0, float)
-        SI_GQA_CHUNK(1, 1, __half)
-        SI_GQA_CHUNK(2, 1, __half)
-        SI_GQA_CHUNK(3, 1, __half)
-        SI_GQA_CHUNK(4, 1, __half)
-#undef SI_GQA_CHUNK
-        default: return hipErrorInvalidValue;
-        }
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess)
-            return e;
-        hipLaunchKernelGGL((gqa_merge_chunks_kernel<128, GQA_FCHUNK>), heads, dim3(128), 0, s, a);
-        return hipGetLastError();
-    }
-#define SI_GQA(T, H)                                                                                              \
-    do {                                                                                                          \
-        hipLaunchKernelGGL((gqa_partial_kernel<T, H>), grid, dim3(GQA_THREADS), 0, s, a,                         \
-                           static_cast<const T*>(a.key_cache), static_cast<const T*>(a.value_cache));            \
-        const hipError_t e = hipGetLastError();                                                                   \
-        if (e != hipSuccess)                                                                                      \
-            return e;                                                                                             \
-        hipLaunchKernelGGL((gqa_merge_kernel<H>), heads, dim3(H), 0, s, a);                                       \
-    } while (0)
+    if (a.kv_heads < 1 || a.query_heads < 1 || a.query_heads % a.kv_heads != 0)
+        return hipErrorInvalidValue;
     switch (a.head_size) {
-    case 64: if (a.cache_fp16) SI_GQA(__half, 64); else SI_GQA(float, 64); break;
-    case 128: if (a.cache_fp16) SI_GQA(__half, 128); else SI_GQA(float, 128); break;
-    case 256: if (a.cache_fp16) SI_GQA(__half, 256); else SI_GQA(float, 256); break;
+    case 64: return a.cache_fp16 ? launch_gqa_head<__half, 64>(a, s) : launch_gqa_head<float, 64>(a, s);
+    case 128: return a.cache_fp16 ? launch_gqa_head<__half, 128>(a, s) : launch_gqa_head<float, 128>(a, s);
+    case 256: return a.cache_fp16 ? launch_gqa_head<__half, 256>(a, s) : launch_gqa_head<float, 256>(a, s);
     default: return hipErrorInvalidValue;
     }
-#undef SI_GQA
-    return hipGetLastError();
 }
 
 }  // namespace si

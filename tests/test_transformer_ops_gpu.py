@@ -166,6 +166,22 @@ def test_grouped_query_attention(hip, fmt, heads, kv_heads, head, context, posit
         assert np.linalg.norm(out - ref) / np.linalg.norm(ref) <= 1e-5
 
 
+# Chunk forms of 64 and 128 rows, groups split into parts (5: 3 + 2 heads),
+# merges of one chunk to several batches, the last row of a chunk and the
+# first of the next.  The tolerance is FP32's: scores of |q.k| / sqrt(head)
+# <= ~6 carry 2^-24 x 6 into the exponentials, the sums a few 2^-24 more.
+@pytest.mark.parametrize("fmt", [native.F32, native.F16], ids=["f32", "f16"])
+@pytest.mark.parametrize("heads,kv_heads,head,context,position",
+                         [(32, 4, 64, 4096, 4000), (5, 1, 64, 1, 0), (10, 2, 64, 65, 64), (4, 4, 64, 511, 63),
+                          (6, 1, 128, 520, 512), (12, 2, 128, 2048, 127), (7, 1, 128, 16384, 16383),
+                          (8, 1, 256, 64, 63), (5, 1, 256, 2049, 2048), (4, 4, 256, 9000, 8999),
+                          (1, 1, 64, 16384, 16000), (40, 8, 64, 2048, 1999)])
+def test_grouped_query_attention_forms(hip, fmt, heads, kv_heads, head, context, position):
+    _, _, _, out, t64, _ = _gqa(hip, fmt, heads, kv_heads, head, context, position, heads + head + position)
+    assert np.linalg.norm(out - t64) / np.linalg.norm(t64) <= 2e-6
+    _close(out, t64, 1e-4, "attention vs fp64")
+
+
 def test_op_rejections(hip):
     buf = hip.alloc(1 << 20)
     p = buf.ptr
