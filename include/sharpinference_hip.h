@@ -126,8 +126,9 @@ int si_hip_sync(si_hip_context* ctx);
 /* y[rows] = W[rows, cols] . x[cols] (+ residual[rows] when residual != NULL),
  * W in GGUF Q8_0 / Q4_0 / Q4_K block layout, x, y, residual FP32.  FP32
  * arithmetic and accumulation.  `path` (optional) receives 1 for the tiled
- * gfx950 kernel, 2 for the any-shape kernel (one wave per row) and 3 for the
- * short-row kernel (rows of at most 32 blocks and 2048 columns, one lane per
+ * gfx950 kernel, 2 for the kernels of any whole number of blocks (streaming,
+ * or one wave per row for weights at odd addresses) and 3 for the short-row
+ * kernel (rows of at most 32 blocks and 2048 columns, one lane per
  * block).
  * Replaces: the core.mat-vec instruction (cooperative form
  * GpuTierZeroInstruction.cs:44-89 on D3D12, CpuInstructionNumerics.MatVec

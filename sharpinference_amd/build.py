@@ -30,6 +30,7 @@ SOURCES = [
     "si_abi.cpp",
     "si_model.cpp",
     "si_gemv.hip",
+    "si_gemv_stream.hip",
     "si_prefill.hip",
     "si_decode.hip",
     "si_rwkv.hip",

@@ -417,3 +417,69 @@ def test_checksum_sums_every_word(hip):
     with pytest.raises(native.HipError):
         hip.checksum(parts.ptr, 6, parts.ptr + 8192)            # not whole words
     parts.free()
+
+
+# ---- the streaming kernel -----------------------------------------------------------------
+
+def _dense(fmt, rows, cols, seed):
+    v = orc.gen_normal_f32(seed, rows * cols, 0.0, 0.02)
+    return (v if fmt == native.F32 else v.astype(np.float16)).view(np.uint8)
+
+
+# one to many steps of the slices, one row to a ragged last workgroup, one and
+# two rows per lane (>= 4096 rows), odd block counts (rows at 2-byte
+# addresses), dense columns past the last 32
+STREAM = [(native.Q8_0, 1, 1056), (native.Q8_0, 4099, 2080), (native.Q8_0, 17, 4160), (native.Q8_0, 9001, 1088),
+          (native.Q4_0, 5, 1056), (native.Q4_0, 4096, 2112), (native.Q4_0, 33, 12000), (native.Q4_0, 8200, 1120),
+          (native.Q4_K, 1, 2304), (native.Q4_K, 5001, 11008), (native.Q4_K, 4097, 2304), (native.Q4_K, 16, 8448),
+          (native.F16, 3, 33), (native.F16, 300, 777), (native.F16, 5, 11007), (native.F16, 1000, 256),
+          (native.F32, 2, 63), (native.F32, 65, 4097), (native.F32, 9, 512)]
+STREAM_NAMES = {**NAMES, native.F16: "f16", native.F32: "f32"}
+
+
+@pytest.mark.parametrize("fmt,rows,cols", STREAM, ids=[f"{STREAM_NAMES[f]}-{r}x{c}" for f, r, c in STREAM])
+def test_streaming_form_matches_oracle(hip, fmt, rows, cols):
+    """Plain product with a residual, x off 16-byte alignment, weights at a
+    2-byte address; SwiGLU rows; one huge, one infinite and one NaN value.
+    FP32 sums of at most 12000 products in 64 partial sums per row: the L2
+    error stays within 2^-24 sqrt(12000 / 64) < 1e-6 of the rows' norm for the
+    products, a few times that through SwiGLU."""
+    w = orc.gen_quant(fmt, 5 + rows, rows, cols) if fmt in NAMES else _dense(fmt, rows, cols, 5 + rows)
+    x = orc.gen_normal_f32(6 + cols, cols)
+    r = orc.gen_normal_f32(7 + cols, rows)
+    dw, dx, dy = hip.alloc(w.nbytes + 2), hip.alloc(4 * cols + 4), hip.alloc(4 * rows)
+    dw.upload(w, offset=2)
+    dr = hip.to_device(r)
+
+    def product(xv):
+        dx.upload(np.ascontiguousarray(xv, np.float32), offset=4)
+        assert hip.gemv(fmt, dw.ptr + 2, dx.ptr + 4, dy.ptr, rows, cols, residual=dr.ptr) == native.PATH_GENERIC
+        return dy.readback(np.float32, rows)
+
+    if rows >= 4:
+        t = orc.gemv_f64(fmt, w, x, rows, cols) + r.astype(np.float64)
+        y = product(x)
+        assert_gemv_close(y, t)
+        assert np.linalg.norm(y - t) / np.linalg.norm(t) <= 2e-6
+        gu = orc.gemv_f64(fmt, w, x, rows, cols)
+        half = rows // 2
+        hip.gemv_batch([native.gemv_op(fmt, dw.ptr + 2, dx.ptr + 4, dy.ptr, half, cols, output=native.OUT_SWIGLU_ROWS)])
+        g, u = gu[:half], gu[half:2 * half]
+        assert_gemv_close(dy.readback(np.float32, half), g / (1 + np.exp(-g)) * u, "swiglu rows")
+    else:
+        assert_gemv_close(product(x), orc.gemv_f64(fmt, w, x, rows, cols) + r.astype(np.float64))
+    wd = (orc.dequant(fmt, w, rows, cols) if fmt in NAMES else
+          w.view(np.float16 if fmt == native.F16 else np.float32)).reshape(rows, cols).astype(np.float64)
+    for at, bad in ((cols - 1, np.float32(3e33)), (cols // 2, np.inf), (31, np.nan)):
+        xb = x.copy()
+        xb[at] = bad
+        y = product(xb)
+        with np.errstate(invalid="ignore", over="ignore"):
+            t = wd @ xb.astype(np.float64) + r
+        assert np.array_equal(np.isnan(y), np.isnan(t))
+        fin = np.isfinite(t)
+        assert np.array_equal(y[~fin & ~np.isnan(t)], t[~fin & ~np.isnan(t)].astype(np.float32))
+        if fin.any():
+            assert_gemv_close(y[fin], t[fin], f"{bad}")
+    for b in (dw, dx, dy, dr):
+        b.free()
