@@ -32,6 +32,7 @@ SOURCES = [
     "si_gemv.hip",
     "si_gemv_stream.hip",
     "si_prefill.hip",
+    "si_prefill_skinny.hip",
     "si_decode.hip",
     "si_rwkv.hip",
     "si_rwkv_program.cpp",

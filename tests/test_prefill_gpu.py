@@ -84,6 +84,41 @@ def test_prefill_matches_oracle(hip, fmt, m, rows, cols):
     check(y, xb @ wb.T, 1e-5, "vs bf16-operand product")
 
 
+# the skinny form: 1 to 4 token tiles and their tails, two and more tiles of 64
+# tokens, 16- and 32-row workgroups with row tails, waves without steps, an
+# odd last block, fewer and more steps than are held in flight
+SKINNY_FORMATS = [native.Q8_0, native.Q4_0, native.Q4_K, native.F16, native.F32]
+SKINNY = [(1, 1, 256), (16, 17, 512), (17, 33, 1280), (48, 100, 256), (49, 16, 8448), (64, 4129, 768), (65, 300, 2304),
+          (130, 1000, 512), (257, 40, 3072)]
+ODD = [(1, 17, 32), (33, 50, 96), (64, 4100, 544), (20, 31, 4128), (129, 65, 1056)]
+SKINNY_CASES = [(f, *c) for f in SKINNY_FORMATS for c in SKINNY + (ODD if f != native.Q4_K else [])]
+SKINNY_NAMES = {**NAMES, native.F16: "f16", native.F32: "f32"}
+
+
+@pytest.mark.parametrize("fmt,m,rows,cols", SKINNY_CASES,
+                         ids=[f"{SKINNY_NAMES[f]}-m{m}-{n}x{k}" for f, m, n, k in SKINNY_CASES])
+def test_skinny_prefill_matches_oracle(hip, fmt, m, rows, cols):
+    """Against the product of the matrix-core operands (FP32 sums of at most
+    8448 products: 1e-5) with rows around Y left alone."""
+    if fmt in NAMES:
+        w = orc.gen_quant(fmt, 50 + rows, rows, cols)
+        wd = orc.dequant(fmt, w, rows, cols).reshape(rows, cols)
+    else:
+        wd = orc.gen_normal_f32(50 + rows, rows * cols, 0.0, 0.02).reshape(rows, cols)
+        wd = wd.astype(np.float16) if fmt == native.F16 else wd
+        w = wd.reshape(-1).view(np.uint8)
+    x = orc.gen_normal_bf16(60 + m, m * cols)
+    dw, dx = hip.to_device(w), hip.to_device(x)
+    dy = hip.to_device(np.full((m + 2) * rows, 13.0, np.float32))
+    hip.gemm_prefill(fmt, dw.ptr, dx.ptr, dy.ptr + 4 * rows, m, rows, cols)
+    y = dy.readback(np.float32, (m + 2) * rows).reshape(m + 2, rows)
+    assert np.all(y[0] == 13.0) and np.all(y[-1] == 13.0)
+    wb = bf16_round(wd.astype(np.float32)).astype(np.float64).reshape(rows, cols)
+    check(y[1:-1], orc.bf16_to_f32(x).reshape(m, cols).astype(np.float64) @ wb.T, 1e-5, "vs bf16-operand product")
+    for b in (dw, dx, dy):
+        b.free()
+
+
 CONFIG4 = [("qkv", 5120, 3072), ("o_proj", 3072, 3072), ("gate_up", 16384, 3072), ("down", 3072, 8192)]
 
 
