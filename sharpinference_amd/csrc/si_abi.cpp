@@ -4,6 +4,7 @@
 #include "si_context.hpp"
 #include "si_decode.hpp"
 
+#include <algorithm>
 #include <vector>
 
 namespace si_abi {
@@ -77,6 +78,72 @@ int check_matrix(si_hip_context* ctx, const char* op, int fmt, const void* w, in
 }  // namespace si_abi
 
 using namespace si_abi;
+
+namespace {
+
+// A plan of a few kernels is launched kernel by kernel: handing a graph to
+// the runtime costs the host about 16 us however few nodes it has, a kernel
+// launch about 3.  Replays back to back, Q8_0 2048 x 2048 products, graph and
+// kernel by kernel: one 16.6 and 3.3 us, two 16.7 and 6.2, four 18.4 and
+// 14.1, six 20.6 and 19.7, eight 24.8 and 28.8.
+constexpr size_t DIRECT_KERNELS = 4;
+
+// The kernel launches of a graph that is one chain of at most DIRECT_KERNELS
+// of them, in order; empty for any other graph.
+std::vector<hipKernelNodeParams> chain_of_kernels(hipGraph_t graph)
+{
+    size_t n = 0, ne = 0;
+    if (hipGraphGetNodes(graph, nullptr, &n) != hipSuccess || n == 0 || n > DIRECT_KERNELS ||
+        hipGraphGetEdges(graph, nullptr, nullptr, &ne) != hipSuccess || ne != n - 1)
+        return {};
+    std::vector<hipGraphNode_t> nodes(n), from(ne), to(ne);
+    if (hipGraphGetNodes(graph, nodes.data(), &n) != hipSuccess || n != nodes.size() ||
+        (ne > 0 && (hipGraphGetEdges(graph, from.data(), to.data(), &ne) != hipSuccess || ne != from.size())))
+        return {};
+    // n nodes and n - 1 edges from node to node without a branch are a chain
+    // when a walk from the one root passes every node
+    hipGraphNode_t at = nullptr;
+    for (hipGraphNode_t v : nodes)
+        if (std::find(to.begin(), to.end(), v) == to.end()) {
+            if (at)
+                return {};
+            at = v;
+        }
+    std::vector<hipKernelNodeParams> out;
+    while (at) {
+        hipGraphNodeType type;
+        hipKernelNodeParams p{};
+        if (hipGraphNodeGetType(at, &type) != hipSuccess || type != hipGraphNodeTypeKernel ||
+            hipGraphKernelNodeGetParams(at, &p) != hipSuccess || !p.func || !p.kernelParams || p.extra)
+            return {};
+        out.push_back(p);
+        hipGraphNode_t next = nullptr;
+        for (size_t e = 0; e < ne; e++)
+            if (from[e] == at) {
+                if (next)
+                    return {};
+                next = to[e];
+            }
+        at = next;
+        if (out.size() > n)
+            return {};
+    }
+    return out.size() == n ? out : std::vector<hipKernelNodeParams>{};
+}
+
+hipError_t launch_plan(const si_hip_plan* plan, hipStream_t s)
+{
+    if (plan->kernels.empty())
+        return hipGraphLaunch(plan->exec, s);
+    for (const hipKernelNodeParams& p : plan->kernels) {
+        const hipError_t e = hipLaunchKernel(p.func, p.gridDim, p.blockDim, p.kernelParams, p.sharedMemBytes, s);
+        if (e != hipSuccess)
+            return e;
+    }
+    return hipSuccess;
+}
+
+}  // namespace
 
 extern "C" {
 
@@ -426,6 +493,8 @@ int si_hip_plan_end(si_hip_context* ctx, si_hip_plan** out)
     plan->ctx = ctx;
     plan->graph = graph;
     plan->exec = exec;
+    plan->kernels = chain_of_kernels(graph);
+    (void)hipGetLastError();   // a graph that cannot be read is launched as a graph
     *out = plan;
     return SI_HIP_OK;
 }
@@ -452,8 +521,8 @@ int si_hip_plan_launch(si_hip_plan* plan)
     Enter g(ctx);
     if (ctx->recording)
         return fail(ctx, SI_HIP_ERR_STATE, "plan_launch: not allowed while recording a plan");
-    const hipError_t e = hipGraphLaunch(plan->exec, ctx->stream);
-    return e == hipSuccess ? SI_HIP_OK : hip_fail(ctx, e, "hipGraphLaunch");
+    const hipError_t e = launch_plan(plan, ctx->stream);
+    return e == hipSuccess ? SI_HIP_OK : hip_fail(ctx, e, "plan launch");
 }
 
 int si_hip_plan_launch_sequence(si_hip_plan* const* plans, int nplans, int64_t steps)
@@ -468,9 +537,9 @@ int si_hip_plan_launch_sequence(si_hip_plan* const* plans, int nplans, int64_t s
     if (ctx->recording)
         return fail(ctx, SI_HIP_ERR_STATE, "plan_launch_sequence: not allowed while recording a plan");
     for (int64_t i = 0; i < steps; i++) {
-        const hipError_t e = hipGraphLaunch(plans[i % nplans]->exec, ctx->stream);
+        const hipError_t e = launch_plan(plans[i % nplans], ctx->stream);
         if (e != hipSuccess)
-            return hip_fail(ctx, e, "hipGraphLaunch");
+            return hip_fail(ctx, e, "plan launch");
     }
     return SI_HIP_OK;
 }
@@ -491,7 +560,7 @@ int si_hip_plan_measure_us(si_hip_plan* plan, int repetitions, double* microseco
         return fail(ctx, SI_HIP_ERR_STATE, "plan_measure: not allowed while a timer_begin is open");
     hipError_t e = hipEventRecord(ctx->t0, ctx->stream);
     for (int i = 0; e == hipSuccess && i < repetitions; i++)
-        e = hipGraphLaunch(plan->exec, ctx->stream);
+        e = launch_plan(plan, ctx->stream);
     if (e == hipSuccess) e = hipEventRecord(ctx->t1, ctx->stream);
     if (e == hipSuccess) e = hipEventSynchronize(ctx->t1);
     float ms = 0.0f;

@@ -9,6 +9,7 @@
 #include <cstdio>
 #include <mutex>
 #include <string>
+#include <vector>
 
 struct si_hip_context {
     int device = 0;
@@ -27,6 +28,9 @@ struct si_hip_plan {
     si_hip_context* ctx = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
+    // the launches of a short plan in order (their arguments belong to
+    // `graph`); empty: the plan is launched as a graph
+    std::vector<hipKernelNodeParams> kernels;
 };
 
 namespace si_abi {

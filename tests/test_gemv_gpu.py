@@ -483,3 +483,42 @@ def test_streaming_form_matches_oracle(hip, fmt, rows, cols):
             assert_gemv_close(y[fin], t[fin], f"{bad}")
     for b in (dw, dx, dy, dr):
         b.free()
+
+
+# ---- plans of a few kernels ---------------------------------------------------------------
+
+@pytest.mark.parametrize("kernels,copy", [(1, False), (2, False), (4, False), (5, False), (1, True), (3, True)])
+def test_short_plans_replay_in_order(hip, kernels, copy):
+    """A recorded chain of products, each reading the one before, and a plan
+    holding a copy: every replay equals the eager calls, with eager work,
+    other plans and synchronisations between, also after the inputs change."""
+    n = 1024
+    w = [hip.to_device(orc.gen_quant(native.Q8_0, 90 + k, n, n)) for k in range(kernels)]
+    bufs = [hip.alloc(4 * n) for _ in range(kernels + 1)]
+    tail = hip.alloc(4 * n)
+
+    def body():
+        for k in range(kernels):
+            hip.gemv(native.Q8_0, w[k].ptr, bufs[k].ptr, bufs[k + 1].ptr, n, n)
+        if copy:
+            hip.copy(tail.ptr, bufs[-1].ptr, 4 * n)
+
+    bufs[0].upload(orc.gen_normal_f32(1, n))
+    plan, other = hip.record(body), hip.record(lambda: hip.fill_u32(bufs[-1].ptr, 0, n))
+    for seed in (1, 2, 3):
+        bufs[0].upload(orc.gen_normal_f32(seed, n))
+        body()
+        want = bufs[-1].readback(np.uint32)
+        for _ in range(3):
+            other.launch()
+            if copy:
+                hip.fill_u32(tail.ptr, 7, n)
+            plan.launch()
+            assert np.array_equal((tail if copy else bufs[-1]).readback(np.uint32), want)
+        other.launch()
+        assert plan.measure_us(3) > 0
+        assert np.array_equal(bufs[-1].readback(np.uint32), want)
+    plan.destroy()
+    other.destroy()
+    for b in w + bufs + [tail]:
+        b.free()
