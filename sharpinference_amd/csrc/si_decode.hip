@@ -114,22 +114,17 @@ __device__ __forceinline__ void unpack8(const uint4& r, float* f)
 }
 
 
-// Once per step: the rotary table of the new position (frequency
-// 1 / base^(2i / R), cos / sin scaled by rope_scale), shared by every layer
-// that attends at that position.
-__device__ __forceinline__ void rope_table(const AttentionArgs& a, int t)
+// The rotary table of the new position (frequency 1 / base^(2i / R), cos /
+// sin scaled by rope_scale): entry t of it into rope[t] and rope[64 + t].
+__device__ __forceinline__ void rope_entry(float* rope, int t, int position, int rotary, float base, float scale)
 {
-    const int P = *a.position;
-    float* rope = a.workspace + att_rope(a.heads, a.max_chunks);
-    if (t < a.rotary_dim / 2) {
-        const float freq = 1.0f / powf(a.rope_base, 2.0f * static_cast<float>(t) / static_cast<float>(a.rotary_dim));
-        const float angle = static_cast<float>(P) * freq;
-        rope[t] = cosf(angle) * a.rope_scale;
-        rope[64 + t] = sinf(angle) * a.rope_scale;
+    if (t < rotary / 2) {
+        const float freq = 1.0f / powf(base, 2.0f * static_cast<float>(t) / static_cast<float>(rotary));
+        const float angle = static_cast<float>(position) * freq;
+        rope[t] = cosf(angle) * scale;
+        rope[64 + t] = sinf(angle) * scale;
     }
 }
-
-__global__ __launch_bounds__(64) void attention_prep_kernel(AttentionArgs a) { rope_table(a, threadIdx.x); }
 
 // The decode step's first launch: the embedding row of the token (every
 // workgroup but the last) and the step's rotary table (the last
@@ -141,8 +136,9 @@ __global__ __launch_bounds__(256) void step_start_kernel(const uint8_t* __restri
 {
     const int gather_blocks = static_cast<int>(gridDim.x) - 1;
     if (static_cast<int>(blockIdx.x) == gather_blocks) {
-        if (threadIdx.x < 64)
-            rope_table(a, threadIdx.x);
+        if (threadIdx.x < 64)   // one table for every layer that attends at this position
+            rope_entry(a.workspace + att_rope(a.heads, a.max_chunks), threadIdx.x, *a.position, a.rotary_dim, a.rope_base,
+                       a.rope_scale);
         return;
     }
     gather_row<FMT>(table, rows, cols, row_bytes, index, out, blockIdx.x, gather_blocks);
@@ -152,100 +148,81 @@ constexpr int MAX_CHUNKS = 256;
 
 // One workgroup per query head merges the chunk partials (m_c, l_c, o_c):
 // out = sum_c o_c e^(m_c - M) / sum_c l_c e^(m_c - M) with M = max_c m_c.
-// Thread (half, d) takes chunks half, half + 2, ... in batches of
-// COMBINE_BATCH, every load of a batch issued together, and merges the
-// batches online; the two halves merge through LDS.  The first batch is
-// written ahead of the position read (slots past the position hold stale
-// partials and are masked), but the compiler issues its loads inside the
-// merge's branch, after the position check: a cache of up to
-// 2 * COMBINE_BATCH chunks costs the position's round trip and one more.
-// (A branch-free merge that keeps them ahead of the position measured
-// slower; merging inside the last partial workgroup needs a device-scope
-// release per workgroup, which writes back the XCD's L2 and costs far more
-// than this launch.)
-constexpr int COMBINE_BATCH = 16;
-
-struct CombineBatch {
-    float m[COMBINE_BATCH], l[COMBINE_BATCH], o[COMBINE_BATCH];
-};
-
-__device__ __forceinline__ void load_combine_batch(const float* src, int base, int max_chunks, int d, CombineBatch& b)
+// SLOTS groups of 128 threads take chunks slot, slot + SLOTS, ... in batches
+// of BATCH, every load of a batch issued together, merge them online, and
+// the slots merge through LDS.  SLOTS * BATCH covers every chunk the grid
+// holds where that is at most 128, so the merge costs one round trip; the
+// first batch (partials past the position are masked) is requested ahead of
+// the position.  Against two slots of 16 requested after it, a call at 16000
+// cached positions over one KV head takes 13.6 us instead of 16.0, at 8000
+// over eight 16.0 instead of 16.9, and a Phi-4 step at 2048 1121 instead of
+// 1129 us.  (Merging inside the last partial workgroup needs a
+// device-scope release per workgroup, which writes back the XCD's L2 and
+// costs far more than this launch.)  The pointers arrive as preloaded scalar
+// arguments; exponentials use the hardware exp2 (__expf), within a few ulp of
+// expf.
+template <int SLOTS, int BATCH>
+__global__ __launch_bounds__(HEAD_DIM * SLOTS) void attention_combine_kernel(const float* __restrict__ workspace,
+                                                                             const int32_t* __restrict__ position,
+                                                                             float* __restrict__ out, int capacity,
+                                                                             int max_chunks, int chunk_size)
 {
-#pragma unroll
-    for (int i = 0; i < COMBINE_BATCH; i++) {
-        const int c = base + 2 * i;
-        const float* p = src + static_cast<int64_t>(c < max_chunks ? c : 0) * PART;
-        b.m[i] = p[0];
-        b.l[i] = p[1];
-        b.o[i] = p[2 + d];
-    }
-}
-
-// Folds the batch's chunks below `chunks` into (m, l, acc).
-__device__ __forceinline__ void merge_combine_batch(const CombineBatch& b, int base, int chunks, float& m, float& l,
-                                                    float& acc)
-{
-    float bm = m;
-#pragma unroll
-    for (int i = 0; i < COMBINE_BATCH; i++)
-        if (base + 2 * i < chunks)
-            bm = fmaxf(bm, b.m[i]);
-    const float r = __expf(m - bm);   // m = -inf before the first batch: r = 0
-    float bl = 0.0f, bo = 0.0f;
-#pragma unroll
-    for (int i = 0; i < COMBINE_BATCH; i++) {
-        if (base + 2 * i < chunks) {
-            const float w = __expf(b.m[i] - bm);
-            bl = fmaf(b.l[i], w, bl);
-            bo = fmaf(b.o[i], w, bo);
-        }
-    }
-    l = fmaf(l, r, bl);
-    acc = fmaf(acc, r, bo);
-    m = bm;
-}
-
-// The pointers arrive as preloaded scalar arguments; exponentials use the
-// hardware exp2 (__expf), within a few ulp of expf.
-__global__ __launch_bounds__(256) void attention_combine_kernel(const float* __restrict__ workspace,
-                                                                const int32_t* __restrict__ position,
-                                                                float* __restrict__ out, int capacity,
-                                                                int max_chunks, int chunk_size)
-{
-    const int h = blockIdx.x, t = threadIdx.x;
-    const int d = t & (HEAD_DIM - 1), half = t >> 7;
+    const int h = blockIdx.x, d = threadIdx.x & (HEAD_DIM - 1);
+    const int slot = __builtin_amdgcn_readfirstlane(threadIdx.x / HEAD_DIM);
     const float* src = workspace + static_cast<int64_t>(h) * max_chunks * PART;
-    CombineBatch b;
-    load_combine_batch(src, half, max_chunks, d, b);
     const int P = *position;
-    if (P < 0 || P >= capacity) {
-        if (t < HEAD_DIM)
-            out[h * HEAD_DIM + t] = __int_as_float(0x7fc00000);   // position outside the cache
-        return;
-    }
-    const int chunks = P / chunk_size + 1;
+    const bool inside = P >= 0 && P < capacity;
+    const int chunks = inside ? P / chunk_size + 1 : 0;
     float m = -INFINITY, l = 0.0f, acc = 0.0f;
-    if (half < chunks)
-        merge_combine_batch(b, half, chunks, m, l, acc);
-    for (int base = half + 2 * COMBINE_BATCH; base < chunks; base += 2 * COMBINE_BATCH) {
-        load_combine_batch(src, base, max_chunks, d, b);
-        merge_combine_batch(b, base, chunks, m, l, acc);
-    }
-    __shared__ float other[HEAD_DIM + 2];
-    if (half == 1) {
-        other[d] = acc;
-        if (d == 0) {
-            other[HEAD_DIM] = m;
-            other[HEAD_DIM + 1] = l;
+    int base = slot;
+    do {
+        float pm[BATCH], pl[BATCH], po[BATCH];
+#pragma unroll
+        for (int i = 0; i < BATCH; i++) {
+            const float* p = src + static_cast<int64_t>(min(base + SLOTS * i, max_chunks - 1)) * PART;
+            pm[i] = p[0];
+            pl[i] = p[1];
+            po[i] = p[2 + d];
         }
+        float bm = m;
+#pragma unroll
+        for (int i = 0; i < BATCH; i++)
+            bm = base + SLOTS * i < chunks ? fmaxf(bm, pm[i]) : bm;
+        const float r = m == -INFINITY ? 0.0f : __expf(m - bm);
+        float bl = 0.0f, bo = 0.0f;
+#pragma unroll
+        for (int i = 0; i < BATCH; i++) {   // partials past the position may hold anything
+            const bool in = base + SLOTS * i < chunks;
+            const float w = in ? __expf(pm[i] - bm) : 0.0f;
+            bl = fmaf(in ? pl[i] : 0.0f, w, bl);
+            bo = fmaf(in ? po[i] : 0.0f, w, bo);
+        }
+        l = fmaf(l, r, bl);
+        acc = fmaf(acc, r, bo);
+        m = bm;
+        base += SLOTS * BATCH;
+    } while (base < chunks);
+    __shared__ float sm[SLOTS], sl[SLOTS], so[SLOTS][HEAD_DIM];
+    so[slot][d] = acc;
+    if (d == 0) {
+        sm[slot] = m;
+        sl[slot] = l;
     }
     __syncthreads();
-    if (half == 0) {
-        const float m1 = other[HEAD_DIM];
-        const float M = fmaxf(m, m1);
-        const float e0 = __expf(m - M), e1 = __expf(m1 - M);   // half 1 without chunks: m1 = -inf, e1 = 0
-        out[h * HEAD_DIM + d] = fmaf(acc, e0, other[d] * e1) / fmaf(l, e0, other[HEAD_DIM + 1] * e1);
+    if (slot != 0)
+        return;
+    float M = sm[0];
+#pragma unroll
+    for (int k = 1; k < SLOTS; k++)
+        M = fmaxf(M, sm[k]);
+    float lsum = 0.0f, o = 0.0f;
+#pragma unroll
+    for (int k = 0; k < SLOTS; k++) {
+        const float e = __expf(sm[k] - M);   // a slot without chunks: m = -inf, e = 0
+        lsum = fmaf(sl[k], e, lsum);
+        o = fmaf(so[k][d], e, o);
     }
+    out[h * HEAD_DIM + d] = inside ? o / lsum : __int_as_float(0x7fc00000);   // NaN: position outside the cache
 }
 
 // One workgroup = one KV head x one chunk of 64 cache positions.  Writes
@@ -255,7 +232,7 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(const float* __r
 // position; then every K and V row of the chunk is requested (16-byte
 // loads, one 8-value slice per lane), and the queries are staged and
 // rotated while those loads are in flight.
-template <int GROUP>
+template <int GROUP, bool TABLE>
 __global__ __launch_bounds__(ATT_THREADS) void attention_partial_kernel(AttentionArgs a)
 {
     constexpr int QPT = (GROUP * HEAD_DIM + ATT_THREADS - 1) / ATT_THREADS;   // query values per thread
@@ -277,7 +254,7 @@ __global__ __launch_bounds__(ATT_THREADS) void attention_partial_kernel(Attentio
     const int ti = t & (HEAD_DIM - 1);
     const float kn = a.qkv[koff + g * HEAD_DIM + ti];
     const float vn = a.qkv[voff + g * HEAD_DIM + ti];
-    const float rp = rope[ti];                // cos at [0, 64), sin at [64, 128)
+    const float rp = TABLE ? 0.0f : rope[ti];   // cos at [0, 64), sin at [64, 128)
 
     const int P = *a.position;                // index of the new token
     if (P < 0 || P >= a.capacity || start > P)
@@ -324,8 +301,11 @@ __global__ __launch_bounds__(ATT_THREADS) void attention_partial_kernel(Attentio
     if (t < HEAD_DIM) {
         knew[t] = kn;
         vnew[t] = vn;
-        rope_s[t] = rp;
+        if (!TABLE)
+            rope_s[t] = rp;
     }
+    if (TABLE)
+        rope_entry(rope_s, t, P, a.rotary_dim, a.rope_base, a.rope_scale);
     __syncthreads();
     const int half_rot = a.rotary_dim / 2;
     for (int i = t; i < GROUP * half_rot; i += ATT_THREADS)
@@ -493,12 +473,19 @@ __device__ __forceinline__ void rotate8(float* own, const float* partner, const 
 // the caller replays it with (a step recorded for a range of positions), so
 // every chunk's K / V rows are requested together with the position instead
 // of after it.
-template <int GROUP, bool BOUNDED>
+// TABLE: the workgroup computes the rotary table itself, under its K / V
+// loads (a call of its own; a decode step computes it once for all layers).
+// The launch this saves was 2.5 us of a 17 us call (24 heads over 8, 8000
+// cached positions: 16.9 -> 13.2 us with the merge below).
+// direct: the output, for a grid of one chunk, which then needs no merge
+// (null otherwise).
+template <int GROUP, bool BOUNDED, bool TABLE>
 __global__ __launch_bounds__(ATT_THREADS) void attention_chunk_kernel(const float* __restrict__ qkv,
                                                                       const int32_t* __restrict__ position,
                                                                       __half* k_cache, __half* v_cache,
                                                                       float* __restrict__ workspace, int capacity,
-                                                                      int rotary, int max_chunks)
+                                                                      int rotary, int max_chunks, float rope_base,
+                                                                      float rope_scale, float* __restrict__ direct)
 {
     // max_chunks: the workspace's partials per head (its 64-position layout);
     // this grid has ceil(capacity / 128) chunks
@@ -530,8 +517,10 @@ __global__ __launch_bounds__(ATT_THREADS) void attention_chunk_kernel(const floa
     load8(kn_row + 8 * dg, kn);
     load8(kn_row + 8 * pdg, knp);
     load8(vn_row + 8 * dg, vn);
-    load8(rope + 8 * tdg, cs);
-    load8(rope + 64 + 8 * tdg, sn);
+    if constexpr (!TABLE) {
+        load8(rope + 8 * tdg, cs);
+        load8(rope + 64 + 8 * tdg, sn);
+    }
 
     // A chunk past the position (or a position outside the cache) loads no
     // cache rows and stores nothing, but runs the same straight-line code:
@@ -558,6 +547,13 @@ __global__ __launch_bounds__(ATT_THREADS) void attention_chunk_kernel(const floa
     }
 
     // 3. rotate the queries and the new key; the new row in fp16
+    if constexpr (TABLE) {
+        __shared__ __align__(16) float table[2 * 64];
+        rope_entry(table, t, P, rotary, rope_base, rope_scale);
+        __syncthreads();
+        load8(table + 8 * tdg, cs);
+        load8(table + 64 + 8 * tdg, sn);
+    }
 #pragma unroll
     for (int h = 0; h < GROUP; h++)
         rotate8(q[h], qp[h], cs, sn, dg, rotary);
@@ -676,6 +672,12 @@ __global__ __launch_bounds__(ATT_THREADS) void attention_chunk_kernel(const floa
                 wm[wave][h] = m[h];
         }
     __syncthreads();
+    const bool whole = valid && P < FCHUNK;   // the grid's one chunk holds every position
+    if (direct && !whole) {                   // position outside the cache (or the one chunk): NaN
+        for (int i = t; i < GROUP * HEAD_DIM; i += ATT_THREADS)
+            direct[g * GROUP * HEAD_DIM + i] = __int_as_float(0x7fc00000);
+        return;
+    }
     if (!valid)
         return;
     const float* red = reinterpret_cast<const float*>(red4);
@@ -691,6 +693,10 @@ __global__ __launch_bounds__(ATT_THREADS) void attention_chunk_kernel(const floa
             const float lw = (wl[w][0][h] + wl[w][2][h]) + (wl[w][1][h] + wl[w][3][h]);
             o = fmaf(ow, f, o);
             lsum = fmaf(lw, f, lsum);
+        }
+        if (direct) {
+            direct[g * GROUP * HEAD_DIM + i] = o / lsum;
+            continue;
         }
         float* dst = workspace + (static_cast<int64_t>(g * GROUP + h) * max_chunks + chunk) * PART;
         dst[2 + d] = o;
@@ -866,22 +872,34 @@ hipError_t launch_step_start(int fmt, const void* table, int64_t rows, int64_t c
     return hipGetLastError();
 }
 
-hipError_t launch_attention_prep(const AttentionArgs& a, hipStream_t s)
+// The merge of a grid of `chunks` chunks, with no more slots and loads than
+// one round trip takes.
+hipError_t launch_combine(const AttentionArgs& a, int limit, int chunks, int chunk_size, hipStream_t s)
 {
-    hipLaunchKernelGGL(attention_prep_kernel, dim3(1), dim3(64), 0, s, a);
+    const dim3 grid(static_cast<unsigned>(a.heads));
+    if (chunks <= 2)
+        hipLaunchKernelGGL((attention_combine_kernel<1, 2>), grid, dim3(HEAD_DIM), 0, s, a.workspace, a.position, a.out,
+                           limit, a.max_chunks, chunk_size);
+    else if (chunks <= 8)
+        hipLaunchKernelGGL((attention_combine_kernel<1, 8>), grid, dim3(HEAD_DIM), 0, s, a.workspace, a.position, a.out,
+                           limit, a.max_chunks, chunk_size);
+    else if (chunks <= 32)
+        hipLaunchKernelGGL((attention_combine_kernel<4, 8>), grid, dim3(4 * HEAD_DIM), 0, s, a.workspace, a.position,
+                           a.out, limit, a.max_chunks, chunk_size);
+    else if (chunks <= 64)
+        hipLaunchKernelGGL((attention_combine_kernel<8, 8>), grid, dim3(8 * HEAD_DIM), 0, s, a.workspace, a.position,
+                           a.out, limit, a.max_chunks, chunk_size);
+    else
+        hipLaunchKernelGGL((attention_combine_kernel<8, 16>), grid, dim3(8 * HEAD_DIM), 0, s, a.workspace, a.position,
+                           a.out, limit, a.max_chunks, chunk_size);
     return hipGetLastError();
 }
 
-hipError_t launch_attention(const AttentionArgs& a, hipStream_t s, bool prep)
+hipError_t launch_attention(const AttentionArgs& a, hipStream_t s, bool own_table)
 {
     if (a.head_dim != HEAD_DIM || a.kv_heads <= 0 || a.heads % a.kv_heads != 0 || a.max_chunks > MAX_CHUNKS ||
         a.rotary_dim > HEAD_DIM)
         return hipErrorInvalidValue;
-    if (prep) {
-        const hipError_t e = launch_attention_prep(a, s);
-        if (e != hipSuccess)
-            return e;
-    }
     const int group = a.heads / a.kv_heads;
     const dim3 grid(static_cast<unsigned>(a.kv_heads), static_cast<unsigned>(a.max_chunks));
     if (a.rotary_dim % 16 == 0) {
@@ -891,47 +909,48 @@ hipError_t launch_attention(const AttentionArgs& a, hipStream_t s, bool prep)
             return hipErrorInvalidValue;
         const dim3 fgrid(static_cast<unsigned>(a.kv_heads), static_cast<unsigned>(bounded ? a.chunk_bound : all));
         // slices of 8 values and their rotary partners are whole
-        switch (group * 2 + (bounded ? 1 : 0)) {
-#define SI_CHUNK(G, B)                                                                                            \
-    case G * 2 + B:                                                                                               \
-        hipLaunchKernelGGL((attention_chunk_kernel<G, B>), fgrid, dim3(ATT_THREADS), 0, s, a.qkv, a.position,     \
-                           a.k_cache, a.v_cache, a.workspace, a.capacity, a.rotary_dim, a.max_chunks);           \
+        if (bounded && own_table)
+            return hipErrorNotSupported;   // bounded grids belong to a step, which has its table
+        float* const direct = fgrid.y == 1 ? a.out : nullptr;
+        switch (group * 4 + (bounded ? 2 : 0) + (own_table ? 1 : 0)) {
+#define SI_CHUNK(G, B, O)                                                                                         \
+    case G * 4 + 2 * B + O:                                                                                       \
+        hipLaunchKernelGGL((attention_chunk_kernel<G, B, O>), fgrid, dim3(ATT_THREADS), 0, s, a.qkv, a.position,  \
+                           a.k_cache, a.v_cache, a.workspace, a.capacity, a.rotary_dim, a.max_chunks,            \
+                           a.rope_base, a.rope_scale, direct);                                                   \
         break;
-        SI_CHUNK(1, 0)
-        SI_CHUNK(2, 0)
-        SI_CHUNK(3, 0)
-        SI_CHUNK(4, 0)
-        SI_CHUNK(1, 1)
-        SI_CHUNK(2, 1)
-        SI_CHUNK(3, 1)
-        SI_CHUNK(4, 1)
+#define SI_CHUNK_FORMS(G) SI_CHUNK(G, 0, 0) SI_CHUNK(G, 0, 1) SI_CHUNK(G, 1, 0)
+        SI_CHUNK_FORMS(1)
+        SI_CHUNK_FORMS(2)
+        SI_CHUNK_FORMS(3)
+        SI_CHUNK_FORMS(4)
+#undef SI_CHUNK_FORMS
 #undef SI_CHUNK
         default: return hipErrorInvalidValue;
         }
         const hipError_t e = hipGetLastError();
-        if (e != hipSuccess)
+        if (e != hipSuccess || direct)
             return e;
         // positions past the chunks of a bounded grid count as outside the cache
         const int limit = bounded ? min(a.capacity, a.chunk_bound * FCHUNK) : a.capacity;
-        hipLaunchKernelGGL(attention_combine_kernel, dim3(static_cast<unsigned>(a.heads)), dim3(256), 0, s, a.workspace,
-                       a.position, a.out, limit, a.max_chunks, FCHUNK);
-        return hipGetLastError();
+        return launch_combine(a, limit, static_cast<int>(fgrid.y), FCHUNK, s);
     }
     if (a.chunk_bound > 0)
         return hipErrorNotSupported;   // the bounded grid is built for rotary widths that are multiples of 16
-    switch (group) {
-    case 1: hipLaunchKernelGGL((attention_partial_kernel<1>), grid, dim3(ATT_THREADS), 0, s, a); break;
-    case 2: hipLaunchKernelGGL((attention_partial_kernel<2>), grid, dim3(ATT_THREADS), 0, s, a); break;
-    case 3: hipLaunchKernelGGL((attention_partial_kernel<3>), grid, dim3(ATT_THREADS), 0, s, a); break;
-    case 4: hipLaunchKernelGGL((attention_partial_kernel<4>), grid, dim3(ATT_THREADS), 0, s, a); break;
+    switch (group * 2 + (own_table ? 1 : 0)) {
+#define SI_PARTIAL(G, O)                                                                              \
+    case G * 2 + O: hipLaunchKernelGGL((attention_partial_kernel<G, O>), grid, dim3(ATT_THREADS), 0, s, a); break;
+    SI_PARTIAL(1, 0) SI_PARTIAL(1, 1)
+    SI_PARTIAL(2, 0) SI_PARTIAL(2, 1)
+    SI_PARTIAL(3, 0) SI_PARTIAL(3, 1)
+    SI_PARTIAL(4, 0) SI_PARTIAL(4, 1)
+#undef SI_PARTIAL
     default: return hipErrorInvalidValue;
     }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess)
         return e;
-    hipLaunchKernelGGL(attention_combine_kernel, dim3(static_cast<unsigned>(a.heads)), dim3(256), 0, s, a.workspace,
-                       a.position, a.out, a.capacity, a.max_chunks, CHUNK);
-    return hipGetLastError();
+    return launch_combine(a, a.capacity, a.max_chunks, CHUNK, s);
 }
 
 hipError_t launch_argmax(const float* values, int64_t n, void* workspace, int32_t* out, hipStream_t s)

@@ -46,15 +46,14 @@ hipError_t attention_scratch(int device, float** out);
 int64_t argmax_workspace_bytes();
 hipError_t launch_gather_row(int fmt, const void* table, int64_t rows, int64_t cols, const int32_t* index, float* out,
                              hipStream_t s);
-// The per-step preparation (rotary table of the position) runs first when
-// `prep`; a program that attends several layers at one position prepares
-// once and passes prep = false afterwards.
-hipError_t launch_attention_prep(const AttentionArgs& a, hipStream_t s);
 // One launch of the decode step's start: launch_gather_row's embedding row
-// and launch_attention_prep's rotary table.
+// and the rotary table of the position, in the attention workspace.
 hipError_t launch_step_start(int fmt, const void* table, int64_t rows, int64_t cols, const int32_t* index, float* out,
                              const AttentionArgs& a, hipStream_t s);
-hipError_t launch_attention(const AttentionArgs& a, hipStream_t s, bool prep = true);
+// own_table: the call computes the position's rotary table itself; a program
+// that attends several layers at one position has launch_step_start do it once
+// and passes false.
+hipError_t launch_attention(const AttentionArgs& a, hipStream_t s, bool own_table = true);
 hipError_t launch_argmax(const float* values, int64_t n, void* workspace, int32_t* out, hipStream_t s);
 
 }  // namespace si

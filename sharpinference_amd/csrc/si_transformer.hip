@@ -333,6 +333,10 @@ __global__ __launch_bounds__(GQA_THREADS) void gqa_chunk_kernel(GqaArgs a, const
             o = fmaf(ow, f, o);
             lsum = fmaf(lw, f, lsum);
         }
+        if (gridDim.y == 1) {   // the cache is one chunk: no merge follows
+            a.output[static_cast<int64_t>(g * group + h0 + h) * HEAD + d] = o / lsum;
+            continue;
+        }
         float* dst = a.workspace + (static_cast<int64_t>(g * group + h0 + h) * a.chunks + chunk) * (HEAD + 2);
         dst[2 + d] = o;
         if (d == 0) {
@@ -416,7 +420,7 @@ hipError_t launch_gqa_form(const GqaArgs& a, int parts, hipStream_t s)
     hipLaunchKernelGGL((gqa_chunk_kernel<T, HEAD, G, CHUNK>), grid, dim3(GQA_THREADS), 0, s, a,
                        static_cast<const T*>(a.key_cache), static_cast<const T*>(a.value_cache));
     const hipError_t e = hipGetLastError();
-    if (e != hipSuccess)
+    if (e != hipSuccess || chunks == 1)
         return e;
     // one round trip for every chunk count of the cache (two at 256-value
     // heads past 64 chunks), with no more slots and loads than that takes
@@ -437,12 +441,12 @@ hipError_t launch_gqa_form(const GqaArgs& a, int parts, hipStream_t s)
 // 128: 8.8 us against 10.0 with 128 rows; 1 KV head, 16384 rows of 128 in
 // FP32: 13.2 against 15.9 with 128 rows only from 512 workgroups); 256-value
 // heads keep 64 (a lane's rows of a 128-row chunk would not fit its
-// registers).
+// registers).  A cache of at most 128 rows is one chunk and needs no merge.
 template <typename T, int HEAD, int G>
 hipError_t launch_gqa_group(const GqaArgs& a, int parts, hipStream_t s)
 {
     if constexpr (HEAD < 256) {
-        if (static_cast<int64_t>(a.kv_heads) * parts * ((a.context + 127) / 128) >= 256)
+        if (a.context <= 128 || static_cast<int64_t>(a.kv_heads) * parts * ((a.context + 127) / 128) >= 256)
             return launch_gqa_form<T, HEAD, G, 128>(a, parts, s);
     }
     return launch_gqa_form<T, HEAD, G, 64>(a, parts, s);

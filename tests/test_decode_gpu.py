@@ -134,12 +134,12 @@ def _attention_case(hip, heads, kv_heads, capacity, position, seed, rotary=96):
     return out, truth, t64.reshape(-1), kg, vg, kk, vv, qkv
 
 
-def _check_attention(heads, kv_heads, capacity, position, rotary, case):
+def _check_attention(heads, kv_heads, capacity, position, rotary, case, l2=5e-5):
     out, truth, t64, kg, vg, kk, vv, qkv = case
     # against the fp64 evaluation of the same operands: the GEMV gates
-    close(out, t64, 1e-3, 5e-5, "attention vs fp64")
+    close(out, t64, 20 * l2, l2, "attention vs fp64")
     # against the oracle's FP32 sequential softmax: both carry FP32 error
-    close(out, truth, 1e-3, 5e-5, "attention vs oracle")
+    close(out, truth, 20 * l2, l2, "attention vs oracle")
     # appended rows: V exactly; K within one fp16 step plus the rotation's
     # FP32 error: pow/cos/sin of two math libraries may differ in the last
     # bit at angles up to `position` radians, and l*cos - r*sin can cancel
@@ -179,6 +179,24 @@ def test_attention_rotary_widths(hip, rotary, position):
     heads, kv_heads, capacity = 24, 8, 1088
     _check_attention(heads, kv_heads, capacity, position, rotary,
                      _attention_case(hip, heads, kv_heads, capacity, position, 300 + position + rotary, rotary))
+
+
+# cache sizes at the edges of the merge's forms: one chunk (no merge), 2, 3 to
+# 8, 9 to 32, 33 to 64 and more chunks of 128 positions, and of 64 (rotary
+# width 40, up to 256 of them: two round trips)
+@pytest.mark.parametrize("rotary", [96, 40])
+@pytest.mark.parametrize("capacity,position", [(1, 0), (128, 127), (129, 128), (256, 100), (257, 256), (1024, 1023),
+                                               (1100, 1099), (4096, 4095), (4200, 4100), (8192, 8191), (8193, 8192),
+                                               (16384, 16383)])
+def test_attention_merge_forms(hip, capacity, position, rotary):
+    # the rotary frequencies of two math libraries may differ in the last bit:
+    # the angles then differ by up to position * 2^-24 rad, which turns the
+    # query (and the scores, of order 1) by as much; on top of the 5e-5 that
+    # short caches are held to
+    heads, kv_heads = 6, 2
+    _check_attention(heads, kv_heads, capacity, position, rotary,
+                     _attention_case(hip, heads, kv_heads, capacity, position, 500 + capacity, rotary),
+                     5e-5 + position * 2.0 ** -24)
 
 
 def test_attention_position_outside_cache_yields_nan_and_writes_nothing(hip):

@@ -175,7 +175,8 @@ def test_grouped_query_attention(hip, fmt, heads, kv_heads, head, context, posit
                          [(32, 4, 64, 4096, 4000), (5, 1, 64, 1, 0), (10, 2, 64, 65, 64), (4, 4, 64, 511, 63),
                           (6, 1, 128, 520, 512), (12, 2, 128, 2048, 127), (7, 1, 128, 16384, 16383),
                           (8, 1, 256, 64, 63), (5, 1, 256, 2049, 2048), (4, 4, 256, 9000, 8999),
-                          (1, 1, 64, 16384, 16000), (40, 8, 64, 2048, 1999)])
+                          (1, 1, 64, 16384, 16000), (40, 8, 64, 2048, 1999), (6, 2, 128, 128, 127), (9, 1, 64, 128, 3),
+                          (4, 2, 128, 129, 128)])
 def test_grouped_query_attention_forms(hip, fmt, heads, kv_heads, head, context, position):
     _, _, _, out, t64, _ = _gqa(hip, fmt, heads, kv_heads, head, context, position, heads + head + position)
     assert np.linalg.norm(out - t64) / np.linalg.norm(t64) <= 2e-6
