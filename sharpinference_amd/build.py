@@ -40,6 +40,7 @@ SOURCES = [
     "si_transformer.hip",
     "si_ops.cpp",
     "si_batch.hip",
+    "si_batch_matvec.hip",
     "si_batch_abi.cpp",
     "si_t0.hip",
     "si_t0_abi.cpp",

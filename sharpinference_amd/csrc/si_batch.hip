@@ -1294,6 +1294,8 @@ hipError_t launch_batch_matvec(int fmt, const void* w, const float* x, float* y,
                                int64_t cols, const int32_t* control, hipStream_t s)
 {
     const dim3 grid(static_cast<unsigned>((rows + 15) / 16), static_cast<unsigned>((batch + 15) / 16));
+    if (!is_block_quant(fmt) && cols % 64 == 0)
+        return launch_batch_matvec_exchange(fmt, w, x, y, batch, rows, cols, control, s);
     const uint8_t* wb = static_cast<const uint8_t*>(w);
     const int64_t rb = row_bytes(fmt, cols);
     const int r = static_cast<int>(rows), c = static_cast<int>(cols);

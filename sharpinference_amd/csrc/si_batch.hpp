@@ -70,4 +70,9 @@ hipError_t launch_batch_select_last(const float* input, float* out, int batch, i
 hipError_t launch_batch_matvec(int fmt, const void* w, const float* x, float* y, int batch, int64_t rows,
                                int64_t cols, const int32_t* control, hipStream_t s);
 
+// The form for F16 / F32 weights with columns % 64 == 0 (si_batch_matvec.hip);
+// weight and x 16-byte aligned.
+hipError_t launch_batch_matvec_exchange(int fmt, const void* w, const float* x, float* y, int batch, int64_t rows,
+                                        int64_t cols, const int32_t* control, hipStream_t s);
+
 }  // namespace si

@@ -164,6 +164,20 @@ def test_batch_matvec(hip, fmt, rows, cols, batch, valid):
         b.free()
 
 
+# F16 / F32 rows of whole 64-column steps: one step (seven waves without
+# any), fewer and more steps a wave than are in flight, 16- and 32-row
+# workgroups with row tails, one live row; and rows that end in half a step
+DENSE_CASES = [(f, *c) for f in (native.F16, native.F32)
+               for c in [(1, 64, 1, 1), (15, 128, 16, 16), (17, 1088, 7, 5), (4097, 640, 16, 16), (4111, 3136, 16, 1),
+                         (300, 8192, 16, 13), (33, 96, 16, 16)]]
+
+
+@pytest.mark.parametrize("fmt,rows,cols,batch,valid", DENSE_CASES,
+                         ids=[f"{f}-{r}x{c}-b{b}v{v}" for f, r, c, b, v in DENSE_CASES])
+def test_batch_matvec_dense_forms(hip, fmt, rows, cols, batch, valid):
+    test_batch_matvec(hip, fmt, rows, cols, batch, valid)
+
+
 def _frequencies(rotary, base):
     i = np.arange(rotary // 2, dtype=np.float32)
     return (np.float32(1) / np.power(np.float32(base), np.float32(2) * i / np.float32(rotary))).astype(np.float32)
