@@ -484,7 +484,7 @@ __global__ __launch_bounds__(THREADS) void batch_gqa_values_partial_kernel(Batch
 
 // Values, second pass: one workgroup per (live row, query head); the chunk
 // partials are requested VALUES_BATCH at a time and added in chunk order.
-constexpr int VALUES_BATCH = 8;
+constexpr int VALUES_BATCH = 16;
 
 __global__ __launch_bounds__(BATCH_HEAD) void batch_gqa_values_reduce_kernel(BatchAttentionArgs a)
 {
@@ -512,8 +512,10 @@ __global__ __launch_bounds__(BATCH_HEAD) void batch_gqa_values_reduce_kernel(Bat
 
 // ---- scores, causal softmax and values in two launches ------------------------------------
 //
-// First pass: one workgroup per (KV head, 64 positions) holding a live
-// position.  The group's scores of the chunk come from the matrix cores as
+// First pass: one workgroup per (KV head, 64 positions, 16 queries of the
+// group) holding a live position; the queries share the chunk's K and V
+// through the caches, and a workgroup's chain is one pass of products.  The
+// scores of the chunk come from the matrix cores as
 // in batch_gqa_scores_kernel (positions past a row's own position, or past
 // the batch's last one, -inf) into an LDS tile; one wave per query turns its
 // row of the tile into exp(s - m), m the row's largest score in the chunk, and
@@ -531,19 +533,38 @@ __global__ __launch_bounds__(THREADS) void batch_gqa_flash_partial_kernel(BatchA
                                                                           const T* __restrict__ kc,
                                                                           const T* __restrict__ vc)
 {
-    __shared__ __align__(16) float tile[BATCH_MAX * BATCH_GROUP_MAX * FLASH_PITCH];
+    __shared__ __align__(16) float tile[16 * FLASH_PITCH];
     const int g = blockIdx.x, chunk = blockIdx.y;
     const int group = a.query_heads / a.kv_heads;
     const int start = a.control[0], valid = min(a.control[1], a.batch);
     const int nq = max(valid, 0) * group;
     const int64_t last = static_cast<int64_t>(start) + valid - 1;
     const int j0 = chunk * BATCH_CHUNK;
-    if (nq == 0 || last < 0 || j0 > last)
-        return;   // the whole workgroup: no live position in this chunk
+    const int p = blockIdx.z;   // the workgroup's queries: 16 p .. 16 p + 15 of the group's nq
+    if (16 * p >= nq || last < 0 || j0 > last)
+        return;   // the whole workgroup: no live position in this chunk, or no such query
     const int jl = static_cast<int>(min(last, static_cast<int64_t>(a.context) - 1));   // last position read
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = lane & 15, c = lane >> 4;
     const int64_t entries = static_cast<int64_t>(a.batch) * a.query_heads;
     const int64_t chunks = (a.context + BATCH_CHUNK - 1) / BATCH_CHUNK;
+    float q[32];
+    {
+        const int qi = min(16 * p + n, nq - 1);   // queries past the live ones repeat the last: not stored
+        const int r = qi / group, h = g * group + qi % group;
+        const float* src = a.query + (static_cast<int64_t>(r) * a.query_heads + h) * BATCH_HEAD + 32 * c;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            load8(src + 8 * i, q + 8 * i);
+    }
+    // keys: position j of this lane, dims 32c .. 32c + 31
+    const int j = j0 + 16 * wave + n;
+    float k[32];
+    {
+        const T* src = kc + (static_cast<int64_t>(min(j, jl)) * a.kv_heads + g) * BATCH_HEAD + 32 * c;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            load8(src + 8 * i, k + 8 * i);
+    }
     // V rows: positions jc + s (s < 16) of lane group c, channels 32 wave + 2n and + 1
     const int jc = j0 + 16 * c;
     float2 v[16];
@@ -556,31 +577,8 @@ __global__ __launch_bounds__(THREADS) void batch_gqa_flash_partial_kernel(BatchA
             v[s] = jc + s <= jl ? f : make_float2(0.0f, 0.0f);
         }
     }
-    // keys: position j of this lane, dims 32c .. 32c + 31
-    const int j = j0 + 16 * wave + n;
-    float k[32];
-    {
-        const T* src = kc + (static_cast<int64_t>(min(j, jl)) * a.kv_heads + g) * BATCH_HEAD + 32 * c;
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-            load8(src + 8 * i, k + 8 * i);
-    }
-    auto load_q = [&](int p, float* q) {
-        const int qi = 16 * p + n;
-        if (qi < nq) {
-            const int r = qi / group, h = g * group + qi % group;
-            const float* src = a.query + (static_cast<int64_t>(r) * a.query_heads + h) * BATCH_HEAD + 32 * c;
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-                load8(src + 8 * i, q + 8 * i);
-        } else {
-#pragma unroll
-            for (int i = 0; i < 32; i++)
-                q[i] = 0.0f;
-        }
-    };
     const float scale = 1.0f / sqrtf(static_cast<float>(BATCH_HEAD));
-    auto score_pass = [&](int p, const float* q) {
+    {
         floatx4 acc = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = {0.0f, 0.0f, 0.0f, 0.0f};   // two product chains
 #pragma unroll
         for (int s = 0; s < 32; s += 2) {
@@ -590,38 +588,19 @@ __global__ __launch_bounds__(THREADS) void batch_gqa_flash_partial_kernel(BatchA
         acc += acc1;
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            const int qi = 16 * p + 4 * c + e;
-            if (qi < nq) {
-                const int64_t active = static_cast<int64_t>(start) + qi / group;
-                tile[qi * FLASH_PITCH + 16 * wave + n] = j <= jl && j <= active ? acc[e] * scale : -INFINITY;
-            }
-        }
-    };
-    const int passes = (nq + 15) / 16;
-    {
-        float q0[32], q1[32];
-        load_q(0, q0);
-        for (int p = 0; p < passes; p += 2) {
-            if (p + 1 < passes)
-                load_q(p + 1, q1);
-            score_pass(p, q0);
-            if (p + 2 < passes)
-                load_q(p + 2, q0);
-            if (p + 1 < passes)
-                score_pass(p + 1, q1);
+            const int64_t active = static_cast<int64_t>(start) + (16 * p + 4 * c + e) / group;
+            tile[(4 * c + e) * FLASH_PITCH + 16 * wave + n] = j <= jl && j <= active ? acc[e] * scale : -INFINITY;
         }
     }
     __syncthreads();
     float* ml = a.workspace + chunks * entries * BATCH_HEAD;   // (m, l) per [chunk][row][head]
-    // four queries a wave at a time (queries wave, wave + 4, ... ), their
-    // reductions interleaved
-    constexpr int SQ = 4;
-    for (int q0 = wave; q0 < nq; q0 += SQ * (THREADS / 64)) {
+    // four queries a wave, their reductions interleaved
+    constexpr int SQ = 16 / (THREADS / 64);
+    {
         float sc[SQ], m[SQ], e[SQ], l[SQ];
 #pragma unroll
         for (int u = 0; u < SQ; u++) {
-            const int qi = q0 + u * (THREADS / 64);
-            sc[u] = qi < nq ? tile[qi * FLASH_PITCH + lane] : -INFINITY;
+            sc[u] = tile[(wave + u * (THREADS / 64)) * FLASH_PITCH + lane];
             m[u] = sc[u];
         }
 #pragma unroll
@@ -637,37 +616,25 @@ __global__ __launch_bounds__(THREADS) void batch_gqa_flash_partial_kernel(BatchA
             l[u] = rows_sum(row_sum<16>(l[u]));
 #pragma unroll
         for (int u = 0; u < SQ; u++) {
-            const int qi = q0 + u * (THREADS / 64);
-            if (qi < nq) {
-                tile[qi * FLASH_PITCH + lane] = e[u];
-                if (lane == 0) {
-                    const int r = qi / group, h = g * group + qi % group;
-                    float* dst = ml + ((static_cast<int64_t>(chunk) * a.batch + r) * a.query_heads + h) * 2;
-                    dst[0] = m[u];
-                    dst[1] = l[u];
-                }
+            const int slot = wave + u * (THREADS / 64), qi = 16 * p + slot;
+            tile[slot * FLASH_PITCH + lane] = e[u];
+            if (lane == 0 && qi < nq) {
+                const int r = qi / group, h = g * group + qi % group;
+                float* dst = ml + ((static_cast<int64_t>(chunk) * a.batch + r) * a.query_heads + h) * 2;
+                dst[0] = m[u];
+                dst[1] = l[u];
             }
         }
     }
     __syncthreads();
-    auto load_p = [&](int p, float* pr) {
-        const int qi = 16 * p + n;
-        if (qi < nq) {
-            const float4* src = reinterpret_cast<const float4*>(tile + qi * FLASH_PITCH + 16 * c);
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float4 f = src[i];
-                pr[4 * i] = f.x; pr[4 * i + 1] = f.y; pr[4 * i + 2] = f.z; pr[4 * i + 3] = f.w;
-            }
-        } else {
-#pragma unroll
-            for (int s = 0; s < 16; s++)
-                pr[s] = 0.0f;
-        }
-    };
-    for (int p = 0; p < passes; p++) {
+    {
         float pr[16];
-        load_p(p, pr);
+        const float4* src = reinterpret_cast<const float4*>(tile + n * FLASH_PITCH + 16 * c);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float4 f = src[i];
+            pr[4 * i] = f.x; pr[4 * i + 1] = f.y; pr[4 * i + 2] = f.z; pr[4 * i + 3] = f.w;
+        }
         floatx4 lo = {0.0f, 0.0f, 0.0f, 0.0f}, hi = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int s = 0; s < 16; s++) {
@@ -1045,9 +1012,9 @@ __device__ __forceinline__ void decode_staged(const uint8_t* row, int b, int g, 
         bytes_to_float(q & 0x0F0F0F0Fu, nl);          // one nibble per byte
         bytes_to_float((q >> 4) & 0x0F0F0F0Fu, nh);
 #pragma unroll
-        for (int e = 0; e < 4; e++) {   // n - 8 and d (n - 8) are exact in FP32
-            w[e] = d * (nl[e] - 8.0f);       // element 4g+e
-            w[4 + e] = d * (nh[e] - 8.0f);   // element 16+4g+e
+        for (int e = 0; e < 4; e++) {   // d (n - 8): every term is exact in FP32
+            w[e] = fmaf(d, nl[e], -8.0f * d);       // element 4g+e
+            w[4 + e] = fmaf(d, nh[e], -8.0f * d);   // element 16+4g+e
         }
     } else {   // Q4_K sub-block j of the super-block (j is the same for the whole wave)
         const int j = b & 7;
@@ -1071,9 +1038,9 @@ __device__ __forceinline__ void decode_staged(const uint8_t* row, int b, int g, 
         bytes_to_float(lo, nl);
         bytes_to_float(hi, nh);
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            w[e] = __fsub_rn(__fmul_rn(d1, nl[e]), m1);
-            w[4 + e] = __fsub_rn(__fmul_rn(d1, nh[e]), m1);
+        for (int e = 0; e < 4; e++) {   // d1 n is exact (17 by 4 bits): one rounding, as the decode's subtraction
+            w[e] = fmaf(d1, nl[e], -m1);
+            w[4 + e] = fmaf(d1, nh[e], -m1);
         }
     }
 }
@@ -1266,8 +1233,8 @@ hipError_t launch_batch_gqa_values(const BatchAttentionArgs& a, hipStream_t s)
 
 hipError_t launch_batch_gqa_attention(const BatchAttentionArgs& a, const void* value_cache, hipStream_t s)
 {
-    const dim3 grid(static_cast<unsigned>(a.kv_heads),
-                    static_cast<unsigned>((a.context + BATCH_CHUNK - 1) / BATCH_CHUNK));
+    const dim3 grid(static_cast<unsigned>(a.kv_heads), static_cast<unsigned>((a.context + BATCH_CHUNK - 1) / BATCH_CHUNK),
+                    static_cast<unsigned>((a.batch * (a.query_heads / a.kv_heads) + 15) / 16));
     if (a.cache_fp16)
         hipLaunchKernelGGL((batch_gqa_flash_partial_kernel<__half>), grid, dim3(THREADS), 0, s, a,
                            static_cast<const __half*>(a.cache), static_cast<const __half*>(value_cache));
