@@ -143,13 +143,18 @@ __global__ __launch_bounds__(PF_THREADS * KS) void prefill_mfma_kernel(const uin
     // W item i of this thread: idx = t + 256 i -> half h = idx % 2, block
     // bo = (idx / 2) % 2 of the step, tile row idx / 4 (4 consecutive lanes
     // cover one row's two blocks)
-    uint32_t wrow[WI];                                    // byte offset of the W row
+    uint32_t woff[WI], qoff[WI];                          // the items' byte offsets in a step
+    const int wh = t & 1, wbo = (t >> 1) & 1;
 #pragma unroll
     for (int i = 0; i < WI; i++) {
         const int r = (t + i * PF_THREADS) >> 2;
-        wrow[i] = static_cast<uint32_t>(min(n0 + r, N - 1)) * static_cast<uint32_t>(row_bytes);
+        const uint32_t row = static_cast<uint32_t>(min(n0 + r, N - 1)) * static_cast<uint32_t>(row_bytes);
+        woff[i] = item_off<FMT>(row, wbo);
+        qoff[i] = item_qoff<FMT>(row, wbo, wh);
     }
-    const int wh = t & 1, wbo = (t >> 1) & 1;
+    // an odd row of blocks: the last step's second block re-reads the first
+    const int odd_step = (nblk & 1) != 0 ? nblk / 2 : -1;
+    const uint32_t wback = FMT == FMT_Q4_K ? 0 : wbo * blk_bytes<FMT>();
 
     f32x16 acc[MT][NT];
 #pragma unroll
@@ -163,10 +168,12 @@ __global__ __launch_bounds__(PF_THREADS * KS) void prefill_mfma_kernel(const uin
     u32x4 xr[D][XL];
     auto load_step = [&](int ls, RawW<FMT> (&wdst)[WI], u32x4 (&xdst_regs)[XL]) {
         const int step = step0 + ls;
-        const int blk = min(BPS * step + wbo, nblk - 1);
+        const uint8_t* base = step_base<FMT, BPS>(W, step);
+        const uint8_t* qbase = step_qbase<FMT, BPS>(base, step);
+        const uint32_t back = step == odd_step ? wback : 0;
 #pragma unroll
         for (int i = 0; i < WI; i++)
-            wdst[i] = load_raw<FMT>(W, wrow[i], blk, wh);
+            wdst[i] = load_item<FMT>(base, qbase, woff[i] - back, qoff[i] - back);
         // columns past K (the second block of a partial last step) re-read
         // the row's last chunk; their MFMAs are skipped
         const int col = min(BPS * 32 * step + xcol, K - 8);
@@ -443,20 +450,26 @@ __global__ __launch_bounds__(2 * PF_THREADS) void prefill_ws_kernel(const uint8_
             xdst[e] = r * 8 + (c ^ ((r >> 1) & 7));
         }
         const uint8_t* xbytes = reinterpret_cast<const uint8_t*>(X);
-        uint32_t wrow[WI];
+        uint32_t woff[WI], qoff[WI];
+        const int wh = t & 1, wbo = (t >> 1) & 1;
 #pragma unroll
         for (int i = 0; i < WI; i++) {
             const int r = (t + i * PF_THREADS) >> 2;
-            wrow[i] = static_cast<uint32_t>(min(n0 + r, N - 1)) * static_cast<uint32_t>(row_bytes);
+            const uint32_t row = static_cast<uint32_t>(min(n0 + r, N - 1)) * static_cast<uint32_t>(row_bytes);
+            woff[i] = item_off<FMT>(row, wbo);
+            qoff[i] = item_qoff<FMT>(row, wbo, wh);
         }
-        const int wh = t & 1, wbo = (t >> 1) & 1;
+        const int odd_step = (nblk & 1) != 0 ? nblk / 2 : -1;   // its second block re-reads the first
+        const uint32_t wback = FMT == FMT_Q4_K ? 0 : wbo * blk_bytes<FMT>();
         RawW<FMT> raw[D][WI];
         u32x4 xr[D][XL];
         auto load_step = [&](int step, RawW<FMT> (&wdst)[WI], u32x4 (&xdst_regs)[XL]) {
-            const int blk = min(BPS * (s0 + step) + wbo, nblk - 1);
+            const uint8_t* base = step_base<FMT, BPS>(W, s0 + step);
+            const uint8_t* qbase = step_qbase<FMT, BPS>(base, s0 + step);
+            const uint32_t back = s0 + step == odd_step ? wback : 0;
 #pragma unroll
             for (int i = 0; i < WI; i++)
-                wdst[i] = load_raw<FMT>(W, wrow[i], blk, wh);
+                wdst[i] = load_item<FMT>(base, qbase, woff[i] - back, qoff[i] - back);
             const int col = min(BPS * 32 * (s0 + step) + xcol, K - 8);
 #pragma unroll
             for (int e = 0; e < XL; e++)
@@ -602,14 +615,16 @@ __global__ __launch_bounds__(PF_THREADS * KS) void prefill_m16_kernel(const uint
     }
     const uint8_t* xbytes = reinterpret_cast<const uint8_t*>(X);
     // W item i: half t % 2 of block (t / 2) % BPS of tile row (t + 256 i) / (2 BPS)
-    uint32_t wrow[WI];
+    uint32_t woff[WI], qoff[WI];
     int wr[WI];
+    const int wh = t & 1, wbo = (t >> 1) % BPS;
 #pragma unroll
     for (int i = 0; i < WI; i++) {
         wr[i] = (t + PF_THREADS * i) / (2 * BPS);
-        wrow[i] = static_cast<uint32_t>(min(n0 + wr[i], N - 1)) * static_cast<uint32_t>(row_bytes);
+        const uint32_t row = static_cast<uint32_t>(min(n0 + wr[i], N - 1)) * static_cast<uint32_t>(row_bytes);
+        woff[i] = item_off<FMT>(row, wbo);
+        qoff[i] = item_qoff<FMT>(row, wbo, wh);
     }
-    const int wh = t & 1, wbo = (t >> 1) % BPS;
 
     f32x4 acc[WM][WN];
 #pragma unroll
@@ -622,10 +637,11 @@ __global__ __launch_bounds__(PF_THREADS * KS) void prefill_m16_kernel(const uint
     u32x4 xr[D][XL];
     auto load_step = [&](int ls, RawW<FMT> (&wd)[WI], u32x4 (&xd)[XL]) {
         const int step = step0 + ls;
-        const int blk = BPS * step + wbo;
+        const uint8_t* base = step_base<FMT, BPS>(W, step);
+        const uint8_t* qbase = step_qbase<FMT, BPS>(base, step);
 #pragma unroll
         for (int i = 0; i < WI; i++)
-            wd[i] = load_raw<FMT>(W, wrow[i], blk, wh);
+            wd[i] = load_item<FMT>(base, qbase, woff[i], qoff[i]);
         const uint32_t col_bytes = static_cast<uint32_t>(64 * BPS * step);
 #pragma unroll
         for (int e = 0; e < XL; e++)
@@ -804,10 +820,14 @@ inline int prefill_splits(int64_t tiles, int64_t steps, int cus, int min_steps)
 //   * up to 64 tokens, or a grid of 32-row x 64-token tiles of at most one to
 //     one and a half per CU (one where K is long enough to be split below):
 //     the skinny form (si_prefill_skinny.hip).  Q8_0 against the choices
-//     below: 16384 x 3072 at 64 tokens 31.8 and 48.7 us, at 65 48.4 and 48.9
-//     (1024 tiles); 3072 x 3072 at 256 24.0 and 31.6 (384 tiles), at 400
-//     35.1 and 31.6 (672); 3072 x 8192 at 128 34.7 and 38.6 (192), at 200
-//     58.0 and 39.7 (384); 300 x 3072 at 512 11.4 and 34.2;
+//     below: 16384 x 3072 at 64 tokens 31.6 and 44.5 us, at 100 53.5 and 45.3
+//     (1024 tiles); 3072 x 3072 at 256 23.9 and 26.6 (384 tiles), at 400
+//     35.0 and 27.1 (672); 3072 x 8192 at 100 32.4 and 33.0 (192), at 200
+//     57.8 and 33.9 (384); 300 x 3072 at 400 10.2 and 25.4.  The figures of
+//     the choices below were taken against each other with word-wide W loads
+//     (the wide loads took all of them further: Q4_K at 2048 tokens 157.8 ->
+//     109.6, 81.9 -> 56.1, 318 -> 234 and 222 -> 130 us for the four
+//     projections, F16 212 -> 94, 108 -> 48, 420 -> 218, 269 -> 117);
 //   * grids of more than 256 workgroups of 256 tokens x 64 rows: the
 //     warp-specialised kernel with 256 x 128 tiles (64 x 128 consumer wave
 //     tiles; gate_up 76 -> 67 us);

@@ -32,56 +32,6 @@ namespace {
 
 constexpr int SK_WAVES = 8;
 
-// 16 or 8 bytes at a 2-byte aligned address, one load.
-struct __attribute__((packed, aligned(2))) words4_a2 {
-    uint32_t w[4];
-};
-struct __attribute__((packed, aligned(2))) words2_a2 {
-    uint32_t w[2];
-};
-
-// Bytes of a 32-column block of a row (Q4_K super-blocks are addressed apart).
-template <int FMT>
-constexpr int blk_bytes() { return FMT == FMT_Q4_0 ? 18 : FMT == FMT_Q8_0 ? 34 : FMT == FMT_F16 ? 64 : 128; }
-
-// load_raw with the widest loads the layout allows: `base` is uniform (the
-// weights plus the step; `qbase` Q4_K's chunk of quant bytes), `off` and
-// `qoff` the lane's 32-bit offsets of the block and of its quant bytes, so an
-// address costs no vector arithmetic.
-template <int FMT>
-__device__ __forceinline__ RawW<FMT> load_item(const uint8_t* base, const uint8_t* qbase, uint32_t off, uint32_t qoff)
-{
-    RawW<FMT> r;
-    off = opaque(off);
-    qoff = opaque(qoff);
-    if constexpr (FMT == FMT_Q4_0) {
-        r.w[0] = ld_u16(base + off);
-        const words2_a2 q = *reinterpret_cast<const words2_a2*>(base + qoff);
-        r.w[1] = q.w[0]; r.w[2] = q.w[1];
-    } else if constexpr (FMT == FMT_Q8_0) {
-        r.w[0] = ld_u16(base + off);
-        const words4_a2 q = *reinterpret_cast<const words4_a2*>(base + qoff);
-        r.w[1] = q.w[0]; r.w[2] = q.w[1]; r.w[3] = q.w[2]; r.w[4] = q.w[3];
-    } else if constexpr (FMT == FMT_Q4_K) {
-        const words4_a2 hd = *reinterpret_cast<const words4_a2*>(base + off);
-        const words4_a2 q = *reinterpret_cast<const words4_a2*>(qbase + qoff);
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            r.w[k] = hd.w[k];
-            r.w[4 + k] = q.w[k];
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < (FMT == FMT_F16 ? 2 : 4); i++) {
-            const words4_a2 q = *reinterpret_cast<const words4_a2*>(base + qoff + 16 * i);
-#pragma unroll
-            for (int k = 0; k < 4; k++)
-                r.w[4 * i + k] = q.w[k];
-        }
-    }
-    return r;
-}
-
 template <int FMT, int MT, int WN>
 __global__ __launch_bounds__(64 * SK_WAVES) void prefill_skinny_kernel(const uint8_t* __restrict__ W,
                                                                        const __bf16* __restrict__ X,
@@ -118,13 +68,9 @@ __global__ __launch_bounds__(64 * SK_WAVES) void prefill_skinny_kernel(const uin
     uint32_t woff[WN], qoff[WN], xoff[MT];
 #pragma unroll
     for (int j = 0; j < WN; j++) {
-        woff[j] = static_cast<uint32_t>(min(n0 + 16 * j + lr, N - 1)) * static_cast<uint32_t>(row_bytes);
-        if constexpr (FMT == FMT_Q4_K) {
-            qoff[j] = woff[j] + 16 * h;
-        } else {
-            woff[j] += blk_bytes<FMT>() * bo;
-            qoff[j] = woff[j] + (FMT == FMT_Q4_0 ? 2 + 8 * h : FMT == FMT_Q8_0 ? 2 + 16 * h : blk_bytes<FMT>() / 2 * h);
-        }
+        const uint32_t row = static_cast<uint32_t>(min(n0 + 16 * j + lr, N - 1)) * static_cast<uint32_t>(row_bytes);
+        woff[j] = item_off<FMT>(row, bo);
+        qoff[j] = item_qoff<FMT>(row, bo, h);
     }
 #pragma unroll
     for (int t = 0; t < MT; t++)
@@ -145,8 +91,8 @@ __global__ __launch_bounds__(64 * SK_WAVES) void prefill_skinny_kernel(const uin
     u32x4 xa[D][MT][2];
     auto load_step = [&](int k, RawW<FMT> (&wd)[WN], u32x4 (&xd)[MT][2]) {
         const int st = s0 + k;
-        const uint8_t* wbase = W + static_cast<int64_t>(FMT == FMT_Q4_K ? (st >> 2) * 144 : st * 2 * blk_bytes<FMT>());
-        const uint8_t* qbase = FMT == FMT_Q4_K ? wbase + 16 + 32 * (st & 3) : wbase;
+        const uint8_t* wbase = step_base<FMT, 2>(W, st);
+        const uint8_t* qbase = step_qbase<FMT, 2>(wbase, st);
         const uint8_t* xbase = xb + static_cast<int64_t>(st) * 128;
         const uint32_t back = odd && k == mine - 1 ? bo : 0;
         const uint32_t wback = FMT == FMT_Q4_K ? 0 : back * blk_bytes<FMT>();

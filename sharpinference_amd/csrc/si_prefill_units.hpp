@@ -27,14 +27,18 @@ struct RawW {
     uint32_t w[FMT == FMT_F32 ? 16 : 8];
 };
 
-typedef uint32_t u32_a2 __attribute__((aligned(2)));   // 4 bytes at a 2-byte aligned address
+// 16 or 8 bytes at a 2-byte aligned address, one load.
+struct __attribute__((packed, aligned(2))) words4_a2 {
+    uint32_t w[4];
+};
+struct __attribute__((packed, aligned(2))) words2_a2 {
+    uint32_t w[2];
+};
 
 __device__ __forceinline__ uint32_t ld_u16(const uint8_t* p)
 {
     return *reinterpret_cast<const unsigned short*>(p);
 }
-__device__ __forceinline__ uint32_t ld_u32_a2(const uint8_t* p) { return *reinterpret_cast<const u32_a2*>(p); }
-__device__ __forceinline__ uint32_t ld_u32(const uint8_t* p) { return *reinterpret_cast<const uint32_t*>(p); }
 
 // Hides a value from the optimiser: keeps a 32-bit lane offset from being
 // widened to 64 bits outside the loop (so loads keep the scalar-base
@@ -46,85 +50,81 @@ __device__ __forceinline__ uint32_t opaque(uint32_t v)
     return v;
 }
 
-// Loads address a block through a workgroup-uniform base (W plus the
-// block's offset in a row) and a 32-bit lane offset (the row's offset), so
-// they use the scalar-base addressing form and need no 64-bit vector
-// address arithmetic.  Item h of a block:
+// Bytes of a 32-column block of a row (Q4_K super-blocks are addressed apart).
+template <int FMT>
+constexpr int blk_bytes() { return FMT == FMT_Q4_0 ? 18 : FMT == FMT_Q8_0 ? 34 : FMT == FMT_F16 ? 64 : 128; }
+
+// A step is BPS (2 or 4) blocks of every row, from a multiple of BPS on.  Its
+// uniform base: the rows' bytes of the step (Q4_K: of its super-block), and
+// for Q4_K the step's first chunk of quant bytes.
+template <int FMT, int BPS>
+__device__ __forceinline__ const uint8_t* step_base(const uint8_t* W, int step)
+{
+    return W + (FMT == FMT_Q4_K ? static_cast<int64_t>((BPS * step) >> 3) * 144
+                                : static_cast<int64_t>(step) * (BPS * blk_bytes<FMT>()));
+}
+template <int FMT, int BPS>
+__device__ __forceinline__ const uint8_t* step_qbase(const uint8_t* base, int step)
+{
+    return FMT == FMT_Q4_K ? base + 16 + 32 * (((BPS * step) & 7) >> 1) : base;
+}
+// A lane's 32-bit offsets from those: block bo (< BPS) of the row at row_off,
+// and item h's quant bytes in it.
+template <int FMT>
+__device__ __forceinline__ uint32_t item_off(uint32_t row_off, int bo)
+{
+    return row_off + (FMT == FMT_Q4_K ? 0 : blk_bytes<FMT>() * bo);
+}
+template <int FMT>
+__device__ __forceinline__ uint32_t item_qoff(uint32_t row_off, int bo, int h)
+{
+    return FMT == FMT_Q4_K ? row_off + 32 * (bo >> 1) + 16 * h
+                           : item_off<FMT>(row_off, bo) +
+                                 (FMT == FMT_Q4_0 ? 2 + 8 * h : FMT == FMT_Q8_0 ? 2 + 16 * h : blk_bytes<FMT>() / 2 * h);
+}
+
+// Item h of a block, with the widest loads the layout allows (one load
+// instruction costs the address unit about a cycle per four lanes of a row
+// whatever its width: loaded word by word, Q4_K items took twice the
+// matrix-core time of a step) and no vector address arithmetic:
 //   Q4_0 {fp16 d; u8 qs[16]}: d and bytes 8h..8h+7 (elements 8h..8h+7 in the
 //        low nibbles, 16+8h..16+8h+7 in the high nibbles);
 //   Q8_0 {fp16 d; int8 q[32]}: d and q[16h..16h+15];
-//   Q4_K {fp16 d, dmin; u8 scales[12]; u8 qs[128]} (16-byte aligned
-//        super-blocks), sub-block j = blk % 8: d | dmin << 16, the three
-//        scale words and the 16 quant bytes of elements 16h..16h+15 (nibble
-//        j % 2 of qs[32 (j / 2) + 16h ..]).
+//   Q4_K {fp16 d, dmin; u8 scales[12]; u8 qs[128]}, sub-block j = blk % 8:
+//        d | dmin << 16, the three scale words and the 16 quant bytes of
+//        elements 16h..16h+15 (nibble j % 2 of qs[32 (j / 2) + 16h ..]);
+//   F16 / F32: elements 16h..16h+15, 8 or 16 words.
 template <int FMT>
-__device__ __forceinline__ RawW<FMT> load_raw(const uint8_t* W, uint32_t row_off, int blk, int h);
-
-template <>
-__device__ __forceinline__ RawW<FMT_Q4_0> load_raw<FMT_Q4_0>(const uint8_t* W, uint32_t row_off, int blk, int h)
+__device__ __forceinline__ RawW<FMT> load_item(const uint8_t* base, const uint8_t* qbase, uint32_t off, uint32_t qoff)
 {
-    const uint8_t* b = W + blk * 18;
-    row_off = opaque(row_off);
-    RawW<FMT_Q4_0> r;
-    r.w[0] = ld_u16(b + row_off);
-    r.w[1] = ld_u32_a2(b + (row_off + 2 + 8 * h));
-    r.w[2] = ld_u32_a2(b + (row_off + 6 + 8 * h));
-    return r;
-}
-
-template <>
-__device__ __forceinline__ RawW<FMT_Q8_0> load_raw<FMT_Q8_0>(const uint8_t* W, uint32_t row_off, int blk, int h)
-{
-    const uint8_t* b = W + blk * 34;
-    row_off = opaque(row_off);
-    RawW<FMT_Q8_0> r;
-    r.w[0] = ld_u16(b + row_off);
+    RawW<FMT> r;
+    off = opaque(off);
+    qoff = opaque(qoff);
+    if constexpr (FMT == FMT_Q4_0) {
+        r.w[0] = ld_u16(base + off);
+        const words2_a2 q = *reinterpret_cast<const words2_a2*>(base + qoff);
+        r.w[1] = q.w[0]; r.w[2] = q.w[1];
+    } else if constexpr (FMT == FMT_Q8_0) {
+        r.w[0] = ld_u16(base + off);
+        const words4_a2 q = *reinterpret_cast<const words4_a2*>(base + qoff);
+        r.w[1] = q.w[0]; r.w[2] = q.w[1]; r.w[3] = q.w[2]; r.w[4] = q.w[3];
+    } else if constexpr (FMT == FMT_Q4_K) {
+        const words4_a2 hd = *reinterpret_cast<const words4_a2*>(base + off);
+        const words4_a2 q = *reinterpret_cast<const words4_a2*>(qbase + qoff);
 #pragma unroll
-    for (int k = 0; k < 4; k++)
-        r.w[1 + k] = ld_u32_a2(b + (row_off + 2 + 16 * h + 4 * k));
-    return r;
-}
-
-template <>
-__device__ __forceinline__ RawW<FMT_Q4_K> load_raw<FMT_Q4_K>(const uint8_t* W, uint32_t row_off, int blk, int h)
-{
-    const uint8_t* b = W + (blk >> 3) * 144;
-    const int j = blk & 7;
-    row_off = opaque(row_off);
-    RawW<FMT_Q4_K> r;
-    r.w[0] = ld_u32(b + row_off);
-    r.w[1] = ld_u32(b + (row_off + 4));
-    r.w[2] = ld_u32(b + (row_off + 8));
-    r.w[3] = ld_u32(b + (row_off + 12));
+        for (int k = 0; k < 4; k++) {
+            r.w[k] = hd.w[k];
+            r.w[4 + k] = q.w[k];
+        }
+    } else {
 #pragma unroll
-    for (int k = 0; k < 4; k++)
-        r.w[4 + k] = ld_u32(b + 16 + 32 * (j >> 1) + (row_off + 16 * h + 4 * k));
-    return r;
-}
-
-// F16 / F32 (dense rows, a "block" is 32 consecutive elements): item h is
-// elements 16h..16h+15, 8 words (F16) or 16 words (F32).
-template <>
-__device__ __forceinline__ RawW<FMT_F16> load_raw<FMT_F16>(const uint8_t* W, uint32_t row_off, int blk, int h)
-{
-    const uint8_t* b = W + blk * 64 + 32 * h;
-    row_off = opaque(row_off);
-    RawW<FMT_F16> r;
+        for (int i = 0; i < (FMT == FMT_F16 ? 2 : 4); i++) {
+            const words4_a2 q = *reinterpret_cast<const words4_a2*>(base + qoff + 16 * i);
 #pragma unroll
-    for (int k = 0; k < 8; k++)
-        r.w[k] = ld_u32(b + (row_off + 4 * k));
-    return r;
-}
-
-template <>
-__device__ __forceinline__ RawW<FMT_F32> load_raw<FMT_F32>(const uint8_t* W, uint32_t row_off, int blk, int h)
-{
-    const uint8_t* b = W + blk * 128 + 64 * h;
-    row_off = opaque(row_off);
-    RawW<FMT_F32> r;
-#pragma unroll
-    for (int k = 0; k < 16; k++)
-        r.w[k] = ld_u32(b + (row_off + 4 * k));
+            for (int k = 0; k < 4; k++)
+                r.w[4 * i + k] = q.w[k];
+        }
+    }
     return r;
 }
 
