@@ -127,9 +127,8 @@ int si_hip_sync(si_hip_context* ctx);
  * W in GGUF Q8_0 / Q4_0 / Q4_K block layout, x, y, residual FP32.  FP32
  * arithmetic and accumulation.  `path` (optional) receives 1 for the tiled
  * gfx950 kernel, 2 for the kernels of any whole number of blocks (streaming,
- * or one wave per row for weights at odd addresses) and 3 for the short-row
- * kernel (rows of at most 32 blocks and 2048 columns, one lane per
- * block).
+ * or one wave per row for weights at odd addresses) and 3 for short rows (at
+ * most 32 blocks and 2048 columns).
  * Replaces: the core.mat-vec instruction (cooperative form
  * GpuTierZeroInstruction.cs:44-89 on D3D12, CpuInstructionNumerics.MatVec
  * CpuInstructionNumerics.cs:16-23 on CpuVm) for block-quantized weights,

@@ -433,7 +433,10 @@ STREAM = [(native.Q8_0, 1, 1056), (native.Q8_0, 4099, 2080), (native.Q8_0, 17, 4
           (native.Q4_0, 5, 1056), (native.Q4_0, 4096, 2112), (native.Q4_0, 33, 12000), (native.Q4_0, 8200, 1120),
           (native.Q4_K, 1, 2304), (native.Q4_K, 5001, 11008), (native.Q4_K, 4097, 2304), (native.Q4_K, 16, 8448),
           (native.F16, 3, 33), (native.F16, 300, 777), (native.F16, 5, 11007), (native.F16, 1000, 256),
-          (native.F32, 2, 63), (native.F32, 65, 4097), (native.F32, 9, 512)]
+          (native.F32, 2, 63), (native.F32, 65, 4097), (native.F32, 9, 512),
+          # short rows from 128 columns on
+          (native.Q8_0, 5, 128), (native.Q8_0, 16001, 512), (native.Q4_0, 33, 992), (native.Q4_K, 8001, 1792),
+          (native.Q4_K, 17, 256)]
 STREAM_NAMES = {**NAMES, native.F16: "f16", native.F32: "f32"}
 
 
@@ -453,7 +456,9 @@ def test_streaming_form_matches_oracle(hip, fmt, rows, cols):
 
     def product(xv):
         dx.upload(np.ascontiguousarray(xv, np.float32), offset=4)
-        assert hip.gemv(fmt, dw.ptr + 2, dx.ptr + 4, dy.ptr, rows, cols, residual=dr.ptr) == native.PATH_GENERIC
+        short = cols // native.BLOCK_ELEMS.get(fmt, 1) <= 32 and cols <= 2048
+        assert hip.gemv(fmt, dw.ptr + 2, dx.ptr + 4, dy.ptr, rows, cols, residual=dr.ptr) == \
+            (native.PATH_SHORT if short else native.PATH_GENERIC)
         return dy.readback(np.float32, rows)
 
     if rows >= 4:
