@@ -2,22 +2,23 @@
 // the tiled kernel (si_gemv.hip) does not take.
 //
 // Any whole number of blocks and any 4-byte aligned x, weights at an even
-// address (the kernel above takes the rest, and the ops pinned to it).
+// address (the byte-by-byte kernels of si_gemv.hip take the rest, and the ops
+// pinned to them).
 // A workgroup of 4 waves: groups of `ks` waves split the units of a row
 // among them, a wave holds 4 row slots of 16 lanes, and lane k of a slot
 // takes unit k of the wave's 16-unit step for RL consecutive rows (a unit is
 // 32 columns, 64 for Q4_K).  Each wave stages the 16 units' x into its own
-// part of LDS with coalesced loads and needs no barrier until the slices' sums meet; the
-// weights and x of the next step are requested before the current one is
-// multiplied.  Columns past the last whole unit (F16 / F32) are taken two
-// per lane by the first slice.
+// part of LDS with coalesced loads and needs no barrier until the slices' sums
+// meet; except for the 4-bit formats, the weights and x of the next step are
+// requested before the current one is multiplied.  Columns past the last whole
+// unit (F16 / F32) are taken two per lane by the first slice.
 //
-// Bound: the FP32 products of the 4-bit formats (about 230 vector
-// instructions per 64 weights), HBM for the others.  The generic kernel reads
+// Bound: the decode and FP32 products of the 4-bit formats (Q4_K about 2.7
+// vector instructions a weight), HBM for the others.  The generic kernel reads
 // byte by byte, a wave a row.  Against it, weights from HBM: Q4_K 5001 x 11008
-// 43.5 -> 11.2 us (2.8 TB/s), Q8_0 16000 x 5120 51 -> 18 us (4.8 TB/s), F16
+// 43.5 -> 12.8 us (2.4 TB/s), Q8_0 16000 x 5120 51 -> 18 us (4.8 TB/s), F16
 // 24000 x 3500 86 -> 32 us (5.2 TB/s), F32 64 x 14000 66 -> 9 us.  With 8
-// waves a workgroup the grids' last wave cost more (Q4_K 17 us, F16 41 us).
+// waves a workgroup the grids' last wave cost more (F16 41 us).
 #include "si_gemv_units.hpp"
 
 namespace si {
@@ -26,7 +27,8 @@ namespace {
 struct __attribute__((packed, aligned(2))) u32x4_a2 {
     uint32_t x, y, z, w;
 };
-typedef uint32_t u32_a2 __attribute__((aligned(2)));
+
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ void ld4_a2(const uint8_t* p, uint32_t* v)
 {
@@ -34,6 +36,15 @@ __device__ __forceinline__ void ld4_a2(const uint8_t* p, uint32_t* v)
     v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
 }
 
+// The unit's product with x is the block decoder's, weight by weight in FP32
+// (factoring the offset out of the block, sum(q x) - 8 sum(x), cancels for an
+// x with a mean: zero-mean weights, x = 1 +- 0.1, Q4_0 992 columns 7.4e-7
+// instead of 1.0e-7, Q4_K 11008 columns 6.6e-7 instead of 1.2e-7).  4-bit
+// values need no conversion each: masked into a 16-bit field they are fp16 (n
+// times 2^-24, or 1024 + n with the exponent's bits set), which v_fma_mix_f32
+// multiplies in FP32.  That takes no more time than one conversion a weight
+// and the sums did (Q4_K 8000 x 1792 6.85 -> 6.25 us, 5001 x 11008 12.3 ->
+// 12.8, Q4_0 16000 x 992 5.6 -> 5.5).
 template <int FMT>
 struct SUnit;
 
@@ -49,7 +60,7 @@ struct SUnit<FMT_Q8_0> {
         ld4_a2(p + 18, q + 4);
     }
     __device__ __forceinline__ void prepare() {}
-    __device__ __forceinline__ float half(int, const float4* x, float) const
+    __device__ __forceinline__ float half(int, const float4* x) const
     {
         float a0 = 0.0f, a1 = 0.0f;
 #pragma unroll
@@ -59,7 +70,6 @@ struct SUnit<FMT_Q8_0> {
         }
         return half_lo(d) * (a0 + a1);
     }
-    __device__ float half_exact(int h, const float4* x) const { return half(h, x, 0.0f); }
 };
 
 template <>
@@ -73,26 +83,27 @@ struct SUnit<FMT_Q4_0> {
         ld4_a2(p + 2, q);
     }
     __device__ __forceinline__ void prepare() {}
-    __device__ __forceinline__ float half(int, const float4* x, float sx) const
+    // d sum((n - 8) x): 1024 + n as fp16 bits, less 1032 (both exact)
+    __device__ __forceinline__ float half(int, const float4* x) const
     {
         float a_lo = 0.0f, a_hi = 0.0f;
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            a_lo = dot4_u8(opaque(q[k] & 0x0f0f0f0fu), x[k], a_lo);
-            a_hi = dot4_u8(opaque(q[k] & 0xf0f0f0f0u), x[4 + k], a_hi);
+            a_lo = dot4(q[k], x[k], a_lo);
+            a_hi = dot4(q[k] >> 4, x[4 + k], a_hi);
         }
-        return half_lo(d) * fmaf(-8.0f, sx, fmaf(a_hi, 0.0625f, a_lo));
+        return half_lo(d) * (a_lo + a_hi);
     }
-    // as QUnit<FMT_Q4_0>::half_exact
-    __device__ float half_exact(int, const float4* x) const
+    // the low nibbles of v's bytes, less 8, times x
+    static __device__ __forceinline__ float dot4(uint32_t v, const float4& x, float a)
     {
-        float a = 0.0f;
-        for (int k = 0; k < 4; k++) {
-            const uint32_t t = q[k] ^ 0x88888888u;
-            a = dot4_i8((t << 4) & 0xf0f0f0f0u, x[k], a);
-            a = dot4_i8(t & 0xf0f0f0f0u, x[4 + k], a);
-        }
-        return (half_lo(d) * 0.0625f) * a;
+        const f16x2 offset = {1032, 1032};
+        const f16x2 e = __builtin_bit_cast(f16x2, (v & 0x000f000fu) | 0x64006400u) - offset;          // bytes 0, 2
+        const f16x2 o = __builtin_bit_cast(f16x2, ((v >> 8) & 0x000f000fu) | 0x64006400u) - offset;   // bytes 1, 3
+        a = fmaf(static_cast<float>(e.x), x.x, a);
+        a = fmaf(static_cast<float>(o.x), x.y, a);
+        a = fmaf(static_cast<float>(e.y), x.z, a);
+        return fmaf(static_cast<float>(o.y), x.w, a);
     }
 };
 
@@ -106,6 +117,24 @@ struct SUnit<FMT_Q4_K> : QUnit<FMT_Q4_K> {
         ld4_a2(p, hd);
         ld4_a2(p + 16 + 32 * chunk, qs);
         ld4_a2(p + 32 + 32 * chunk, qs + 4);
+    }
+    // sum(w x) with w = d1 n - m1: d1 n is exact, so the one rounding of the
+    // fused form is the decoder's (its scale carries the nibble's 2^24 or 2^20)
+    __device__ __forceinline__ float half(int h, const float4* x) const
+    {
+        const float scale = dsc[h] * (h == 0 ? 0x1p24f : 0x1p20f), m1 = -dmn[h];
+        const uint32_t mask = h == 0 ? 0x000f000fu : 0x00f000f0u;
+        float a0 = 0.0f, a1 = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const f16x2 e = __builtin_bit_cast(f16x2, qs[k] & mask);          // bytes 0, 2
+            const f16x2 o = __builtin_bit_cast(f16x2, (qs[k] >> 8) & mask);   // bytes 1, 3
+            a0 = fmaf(fmaf(static_cast<float>(e.x), scale, m1), x[k].x, a0);
+            a1 = fmaf(fmaf(static_cast<float>(o.x), scale, m1), x[k].y, a1);
+            a0 = fmaf(fmaf(static_cast<float>(e.y), scale, m1), x[k].z, a0);
+            a1 = fmaf(fmaf(static_cast<float>(o.y), scale, m1), x[k].w, a1);
+        }
+        return a0 + a1;
     }
 };
 
@@ -121,7 +150,7 @@ struct SUnit<FMT_F16> {
             ld4_a2(p + 16 * i, v + 4 * i);
     }
     __device__ __forceinline__ void prepare() {}
-    __device__ __forceinline__ float half(int, const float4* x, float) const
+    __device__ __forceinline__ float half(int, const float4* x) const
     {
         float a0 = 0.0f, a1 = 0.0f;
 #pragma unroll
@@ -147,7 +176,7 @@ struct SUnit<FMT_F32> {
             ld4_a2(p + 16 * i, v + 4 * i);
     }
     __device__ __forceinline__ void prepare() {}
-    __device__ __forceinline__ float half(int, const float4* x, float) const
+    __device__ __forceinline__ float half(int, const float4* x) const
     {
         float a0 = 0.0f, a1 = 0.0f;
 #pragma unroll
@@ -169,16 +198,14 @@ __global__ __launch_bounds__(64 * STREAM_WAVES) void gemv_stream_kernel(Segs<NS>
     using U = SUnit<FMT>;
     constexpr int HALVES = U::COLS / 32;              // 32-column blocks per unit
     constexpr int XPT = U::COLS / 16;                 // float4 values of x per lane and step
-    constexpr bool SUMS = FMT == FMT_Q4_0 || FMT == FMT_Q4_K;
     constexpr bool DENSE = block_elems(FMT) == 1;
     // the 4-bit formats decode long enough for the other waves to cover a
-    // step's round trip, and the registers of a second step would halve
-    // their number (Q4_K 5001 x 11008: 14.8 us ahead, 11.2 without; F16
-    // 24000 x 3500: 32.3 ahead, 33.7 without)
-    constexpr bool AHEAD = !SUMS;
+    // step's round trip, and the registers of a second step cost waves (Q4_K
+    // 20000 x 5120: 24.9 us ahead, 17.9 without; Q4_0 8000 x 5120: 9.9 and
+    // 10.2; F16 24000 x 3500: 32.3 ahead, 33.7 without)
+    constexpr bool AHEAD = FMT != FMT_Q4_0 && FMT != FMT_Q4_K;
     constexpr int XU = 8 * HALVES + 1;                 // float4 values of a unit in LDS, odd: 16 lanes hit distinct banks
     __shared__ float4 xs[STREAM_WAVES][16 * XU];
-    __shared__ float bs[STREAM_WAVES][SUMS ? 16 * HALVES : 1];
     __shared__ float part[2][STREAM_WAVES * 4 * RL];
 
     const Seg& sg = segs.s[NS == 1 ? 0 : blockIdx.y];   // the op of this grid row
@@ -234,15 +261,6 @@ __global__ __launch_bounds__(64 * STREAM_WAVES) void gemv_stream_kernel(Segs<NS>
             for (int j = 0; j < XPT; j++) {
                 const int q = lane + 64 * j;
                 xs[wave][q / (8 * HALVES) * XU + q % (8 * HALVES)] = xd[j];
-                if constexpr (SUMS) {
-                    // a block with a non-finite or huge value stores NaN: the per-weight form
-                    const bool wide = !(fabsf(xd[j].x) <= 0x1p100f && fabsf(xd[j].y) <= 0x1p100f &&
-                                        fabsf(xd[j].z) <= 0x1p100f && fabsf(xd[j].w) <= 0x1p100f);
-                    const float sum =
-                        group_sum<8>(wide ? __builtin_nanf("") : (xd[j].x + xd[j].y) + (xd[j].z + xd[j].w));
-                    if ((lane & 7) == 0)
-                        bs[wave][q >> 3] = sum;
-                }
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             __builtin_amdgcn_wave_barrier();
@@ -256,24 +274,10 @@ __global__ __launch_bounds__(64 * STREAM_WAVES) void gemv_stream_kernel(Segs<NS>
 #pragma unroll
                 for (int k = 0; k < 8; k++)
                     xv[k] = xs[wave][lk * XU + 8 * h + k];
-                if constexpr (SUMS) {
-                    const float sx = bs[wave][lk * HALVES + h];
-                    if (__builtin_expect(sx == sx, 1)) {
 #pragma unroll
-                        for (int t = 0; t < RL; t++) {
-                            const float v = wd[t].half(h, xv, sx);
-                            acc[t] += in ? v : 0.0f;
-                        }
-                    } else if (in) {
-                        for (int t = 0; t < RL; t++)
-                            acc[t] += wd[t].half_exact(h, xv);
-                    }
-                } else {
-#pragma unroll
-                    for (int t = 0; t < RL; t++) {
-                        const float v = wd[t].half(h, xv, 0.0f);
-                        acc[t] += in ? v : 0.0f;
-                    }
+                for (int t = 0; t < RL; t++) {
+                    const float v = wd[t].half(h, xv);
+                    acc[t] += in ? v : 0.0f;
                 }
             }
         };

@@ -490,6 +490,39 @@ def test_streaming_form_matches_oracle(hip, fmt, rows, cols):
         b.free()
 
 
+def _zero_mean_4bit(fmt, rows, cols, seed):
+    """Blocks whose offset lies at the nibbles' middle, as quantised weights
+    have it: Q4_0 n - 8; Q4_K dmin = 7.5 d and equal scale and min."""
+    rng = np.random.default_rng(seed)
+    nib = rng.integers(1 if fmt == native.Q4_0 else 0, 16, rows * cols)
+    if fmt == native.Q4_0:
+        return blocks.q4_0(rng.uniform(0.001, 0.003, rows * cols // 32), nib)
+    nb = rows * cols // 256
+    d, sc = rng.uniform(1e-4, 2e-4, nb).astype(np.float16).astype(np.float64), rng.integers(8, 64, (nb, 8))
+    return blocks.q4_k(d, 7.5 * d, sc, sc, nib)
+
+
+MEANS = [(native.Q4_0, 300, 992), (native.Q4_0, 301, 256), (native.Q4_0, 300, 12000), (native.Q4_0, 4100, 2112),
+         (native.Q4_K, 300, 1792), (native.Q4_K, 300, 11008), (native.Q4_K, 4100, 2304)]
+
+
+@pytest.mark.parametrize("fmt,rows,cols", MEANS, ids=[f"{NAMES[f]}-{r}x{c}" for f, r, c in MEANS])
+def test_streaming_form_keeps_fp32_accuracy_for_x_with_a_mean(hip, fmt, rows, cols):
+    """relu^2 activations and x near 1 (sigmoid values), where a block's
+    sum(q x) is many times the product.  u = 2^-24: chains of 16 products
+    round with variance u^2 / 3 x the partial sum's (1.7 u over the row's
+    standard deviation), the sums over units, lanes and slices (at most 6 + 4 +
+    4 additions of growing partial sums) add at most about as much again: 4 u."""
+    w = _zero_mean_4bit(fmt, rows, cols, rows + cols)
+    n = orc.gen_normal_f32(8 + cols, cols)
+    for name, x in (("normal", n), ("relu^2", np.maximum(n, 0) ** 2), ("near 1", 1 + np.float32(0.1) * n)):
+        y, path = run_gemv(hip, fmt, w, x, rows, cols)
+        assert path != native.PATH_FAST
+        t = orc.gemv_f64(fmt, w, x, rows, cols)
+        l2 = np.linalg.norm(y - t) / np.linalg.norm(t)
+        assert l2 <= 4 * 2.0 ** -24, f"{name}: {l2:.2e}"
+
+
 # ---- plans of a few kernels ---------------------------------------------------------------
 
 @pytest.mark.parametrize("kernels,copy", [(1, False), (2, False), (4, False), (5, False), (1, True), (3, True)])
