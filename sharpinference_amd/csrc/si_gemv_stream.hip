@@ -138,6 +138,14 @@ struct SUnit<FMT_Q4_K> : QUnit<FMT_Q4_K> {
     }
 };
 
+// The dense units' eight chains of four products: as short as the wave a row
+// of the any-shape kernel has them at a few hundred columns (F16, 260 columns:
+// 7.7e-8, with two chains of 16 9.2e-8).
+__device__ __forceinline__ float sum8(const float (&a)[8])
+{
+    return ((a[0] + a[4]) + (a[1] + a[5])) + ((a[2] + a[6]) + (a[3] + a[7]));
+}
+
 template <>
 struct SUnit<FMT_F16> {
     static constexpr int COLS = 32, BYTES = 64;
@@ -152,15 +160,16 @@ struct SUnit<FMT_F16> {
     __device__ __forceinline__ void prepare() {}
     __device__ __forceinline__ float half(int, const float4* x) const
     {
-        float a0 = 0.0f, a1 = 0.0f;
+        float a[8] = {};
 #pragma unroll
         for (int k = 0; k < 8; k++) {
-            a0 = fmaf(half_lo(v[2 * k]), x[k].x, a0);
-            a1 = fmaf(half_hi(v[2 * k]), x[k].y, a1);
-            a0 = fmaf(half_lo(v[2 * k + 1]), x[k].z, a0);
-            a1 = fmaf(half_hi(v[2 * k + 1]), x[k].w, a1);
+            const int c = 4 * (k & 1);
+            a[c] = fmaf(half_lo(v[2 * k]), x[k].x, a[c]);
+            a[c + 1] = fmaf(half_hi(v[2 * k]), x[k].y, a[c + 1]);
+            a[c + 2] = fmaf(half_lo(v[2 * k + 1]), x[k].z, a[c + 2]);
+            a[c + 3] = fmaf(half_hi(v[2 * k + 1]), x[k].w, a[c + 3]);
         }
-        return a0 + a1;
+        return sum8(a);
     }
 };
 
@@ -178,15 +187,16 @@ struct SUnit<FMT_F32> {
     __device__ __forceinline__ void prepare() {}
     __device__ __forceinline__ float half(int, const float4* x) const
     {
-        float a0 = 0.0f, a1 = 0.0f;
+        float a[8] = {};
 #pragma unroll
         for (int k = 0; k < 8; k++) {
-            a0 = fmaf(__uint_as_float(v[4 * k]), x[k].x, a0);
-            a1 = fmaf(__uint_as_float(v[4 * k + 1]), x[k].y, a1);
-            a0 = fmaf(__uint_as_float(v[4 * k + 2]), x[k].z, a0);
-            a1 = fmaf(__uint_as_float(v[4 * k + 3]), x[k].w, a1);
+            const int c = 4 * (k & 1);
+            a[c] = fmaf(__uint_as_float(v[4 * k]), x[k].x, a[c]);
+            a[c + 1] = fmaf(__uint_as_float(v[4 * k + 1]), x[k].y, a[c + 1]);
+            a[c + 2] = fmaf(__uint_as_float(v[4 * k + 2]), x[k].z, a[c + 2]);
+            a[c + 3] = fmaf(__uint_as_float(v[4 * k + 3]), x[k].w, a[c + 3]);
         }
-        return a0 + a1;
+        return sum8(a);
     }
 };
 

@@ -523,6 +523,25 @@ def test_streaming_form_keeps_fp32_accuracy_for_x_with_a_mean(hip, fmt, rows, co
         assert l2 <= 4 * 2.0 ** -24, f"{name}: {l2:.2e}"
 
 
+@pytest.mark.parametrize("fmt", [native.F16, native.F32], ids=["f16", "f32"])
+@pytest.mark.parametrize("cols", [256, 260, 500])
+def test_streaming_dense_rows_sum_in_short_chains(hip, fmt, cols):
+    """A rounding's relative variance is u^2 / 3 E[1 / m^2] = 0.18 u^2 for
+    log-uniform mantissas m in [1, 2), u = 2^-24, and every level of a sum of
+    independent terms adds it once (a chain of n, (n + 1) / 2 times).  Chains of
+    4, their three levels, four of lanes and up to one of slices: 10.5 levels
+    at most, 1.4 u; chains of 16 would make 13.5, 1.56 u."""
+    rows, squares = 300, []
+    for seed in range(16):
+        w = _dense(fmt, rows, cols, 40 + seed)
+        x = orc.gen_normal_f32(70 + seed, cols)
+        y, path = run_gemv(hip, fmt, w, x, rows, cols)
+        assert path == native.PATH_GENERIC
+        t = orc.gemv_f64(fmt, w, x, rows, cols)
+        squares.append(np.sum((y - t) ** 2) / np.sum(t * t))
+    assert np.sqrt(np.mean(squares)) <= 1.47 * 2.0 ** -24
+
+
 # ---- plans of a few kernels ---------------------------------------------------------------
 
 @pytest.mark.parametrize("kernels,copy", [(1, False), (2, False), (4, False), (5, False), (1, True), (3, True)])
