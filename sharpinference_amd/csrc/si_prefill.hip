@@ -819,15 +819,21 @@ inline int prefill_splits(int64_t tiles, int64_t steps, int cus, int min_steps)
 // Tile choice (measured on the Phi-4-mini projections at 512 tokens):
 //   * up to 64 tokens, or a grid of 32-row x 64-token tiles of at most one to
 //     one and a half per CU (one where K is long enough to be split below):
-//     the skinny form (si_prefill_skinny.hip).  Q8_0 against the choices
-//     below: 16384 x 3072 at 64 tokens 31.6 and 44.5 us, at 100 53.5 and 45.3
-//     (1024 tiles); 3072 x 3072 at 256 23.9 and 26.6 (384 tiles), at 400
-//     35.0 and 27.1 (672); 3072 x 8192 at 100 32.4 and 33.0 (192), at 200
-//     57.8 and 33.9 (384); 300 x 3072 at 400 10.2 and 25.4.  The figures of
-//     the choices below were taken against each other with word-wide W loads
-//     (the wide loads took all of them further: Q4_K at 2048 tokens 157.8 ->
-//     109.6, 81.9 -> 56.1, 318 -> 234 and 222 -> 130 us for the four
-//     projections, F16 212 -> 94, 108 -> 48, 420 -> 218, 269 -> 117);
+//     the skinny form (si_prefill_skinny.hip).  It and the choices below, us,
+//     for Q8_0 | Q4_0 | Q4_K | F16 | F32:
+//       16384 x 3072, 64 tokens   25.9 42.4 | 22.9 39.8 | 24.0 40.2 | 30.9 41.2 | 49.5 52.2
+//       3072 x 8192, 64 tokens    20.3 30.7 | 18.3 29.2 | 17.6 29.4 | 17.4 25.6 | 34.8 33.7
+//       3072 x 3072, 256 (384)    23.7 26.2 | 21.6 20.5 | 21.5 21.9 | 20.2 18.9 | 28.8 30.9
+//       3072 x 8192, 100 (192)    27.2 30.9 | 24.2 28.2 | 21.9 28.5 | 20.4 25.8 | 38.5 33.5
+//       2048 x 8192, 256 (256)    27.7 29.6 | 24.8 26.7 | 24.1 27.2 | 21.3 24.1 | 29.4 27.1
+//       300 x 3072, 400 (70)      10.2 25.1 |  9.6 22.8 |  9.7 21.8 |  9.5 19.5 | 12.0 25.8
+//     (tiles in brackets); past the line, Q8_0 3072 x 3072 at 400 tokens (672)
+//     35.0 and 27.1, 3072 x 8192 at 200 (384) 57.8 and 33.9, 16384 x 3072 at 100
+//     (1024) 53.5 and 45.3.  The figures of the choices below were taken against
+//     each other with word-wide W loads (the wide loads took all of them
+//     further: Q4_K at 2048 tokens 157.8 -> 109.6, 81.9 -> 56.1, 318 -> 234 and
+//     222 -> 130 us for the four projections, F16 212 -> 94, 108 -> 48, 420 ->
+//     218, 269 -> 117);
 //   * grids of more than 256 workgroups of 256 tokens x 64 rows: the
 //     warp-specialised kernel with 256 x 128 tiles (64 x 128 consumer wave
 //     tiles; gate_up 76 -> 67 us);

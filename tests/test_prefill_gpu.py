@@ -119,6 +119,19 @@ def test_skinny_prefill_matches_oracle(hip, fmt, m, rows, cols):
         b.free()
 
 
+# X and W of as nearly the same bytes as the format allows: W just the larger
+# (its row tiles side by side in the grid) and X just the larger (the token
+# tiles); one token tile of many row tiles and the other way round
+ORDERS = [(native.Q8_0, 130, 244), (native.Q8_0, 130, 245), (native.Q4_0, 130, 462), (native.Q4_0, 130, 463),
+          (native.Q4_K, 130, 462), (native.Q4_K, 130, 463), (native.F16, 130, 129), (native.F16, 130, 130),
+          (native.F32, 130, 64), (native.F32, 130, 65), (native.Q8_0, 2047, 1), (native.Q4_0, 1, 2047)]
+
+
+@pytest.mark.parametrize("fmt,m,rows", ORDERS, ids=[f"{SKINNY_NAMES[f]}-m{m}-{n}" for f, m, n in ORDERS])
+def test_skinny_prefill_in_both_grid_orders(hip, fmt, m, rows):
+    test_skinny_prefill_matches_oracle(hip, fmt, m, rows, 768)
+
+
 CONFIG4 = [("qkv", 5120, 3072), ("o_proj", 3072, 3072), ("gate_up", 16384, 3072), ("down", 3072, 8192)]
 
 
