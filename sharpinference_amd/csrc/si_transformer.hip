@@ -244,7 +244,8 @@ __global__ __launch_bounds__(GQA_THREADS) void gqa_chunk_kernel(GqaArgs a, const
         }
     }
     // scores q.k / sqrt(HEAD), masked past the count; exponentials with the
-    // hardware exp2 (__expf)
+    // hardware exp2 (__expf: L2 error against 64 bits as with expf to two
+    // digits, for scores of standard deviation 1, 4 and 16; expf costs 6 to 15%)
     const float rscale = 1.0f / sqrtf(static_cast<float>(HEAD));
     float sc[G][PPL];
 #pragma unroll
@@ -352,11 +353,17 @@ __global__ __launch_bounds__(GQA_THREADS) void gqa_chunk_kernel(GqaArgs a, const
 // turn, each a batch of BATCH chunks per round trip merged online (m, l, o
 // rescaled per batch), and merge through LDS: up to BATCH * SLOTS chunks
 // cost one round trip, the first batch's requested before the position is
-// known.
+// known.  Lane u (mod BATCH) holds (m, l) of the batch's chunk u, so a wave
+// issues BATCH + 2 loads for it and not 3 BATCH: 48 loads of 16 waves held the
+// address unit for longer than the merge of a few chunks needs (168 of 2800
+// rows, 6 heads of 128 over 2: 9.4 us a call, 7.5 now; 16383 of 16384, 16 over
+// 4: 17.4, 15.8 now).
 template <int HEAD, int CHUNK, int SLOTS, int BATCH>
 __global__ __launch_bounds__(HEAD * SLOTS) void gqa_merge_kernel(GqaArgs a)
 {
-    const int head = blockIdx.x, d = threadIdx.x % HEAD, slot = threadIdx.x / HEAD;
+    static_assert(HEAD % 64 == 0 && BATCH <= 16, "a slot is whole waves, a batch's (m, l) one row of lanes");
+    const int head = blockIdx.x, d = threadIdx.x % HEAD, own = threadIdx.x % BATCH;
+    const int slot = __builtin_amdgcn_readfirstlane(threadIdx.x / HEAD);
     const float* src = a.workspace + static_cast<int64_t>(head) * a.chunks * (HEAD + 2);
     const int all = (a.context + CHUNK - 1) / CHUNK;   // partials a full cache has
     const int active = min(max(*a.position, 0), a.context - 1);
@@ -364,27 +371,22 @@ __global__ __launch_bounds__(HEAD * SLOTS) void gqa_merge_kernel(GqaArgs a)
     float m = -INFINITY, L = 0.0f, O = 0.0f;
     int c0 = slot;
     do {   // the first batch's loads (any partial of the workspace) need no position
-        float mc[BATCH], lc[BATCH], oc[BATCH];
-#pragma unroll
-        for (int u = 0; u < BATCH; u++) {
-            const float* pc = src + static_cast<int64_t>(min(c0 + u * SLOTS, all - 1)) * (HEAD + 2);
-            mc[u] = pc[0];
-            lc[u] = pc[1];
-            oc[u] = pc[2 + d];
-        }
-        float bm = m;
+        const float* pc = src + static_cast<int64_t>(min(c0 + own * SLOTS, all - 1)) * (HEAD + 2);
+        const float mc = pc[0], lc = pc[1];
+        float oc[BATCH];
 #pragma unroll
         for (int u = 0; u < BATCH; u++)
-            bm = c0 + u * SLOTS < n ? fmaxf(bm, mc[u]) : bm;
+            oc[u] = src[static_cast<int64_t>(min(c0 + u * SLOTS, all - 1)) * (HEAD + 2) + 2 + d];
+        const bool in = c0 + own * SLOTS < n;   // partials past the active chunks may hold anything
+        const float bm = fmaxf(m, row_max<BATCH>(in ? mc : -INFINITY));
         const float r = m == -INFINITY ? 0.0f : __expf(m - bm);
-        L *= r;
+        const float e = in ? __expf(mc - bm) : 0.0f;
+        L = fmaf(L, r, row_sum<BATCH>(in ? lc * e : 0.0f));
         O *= r;
 #pragma unroll
-        for (int u = 0; u < BATCH; u++) {   // partials past the active chunks may hold anything
-            const bool in = c0 + u * SLOTS < n;
-            const float e = in ? __expf(mc[u] - bm) : 0.0f;
-            L = fmaf(in ? lc[u] : 0.0f, e, L);
-            O = fmaf(in ? oc[u] : 0.0f, e, O);
+        for (int u = 0; u < BATCH; u++) {
+            const float eu = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e), u));
+            O = fmaf(c0 + u * SLOTS < n ? oc[u] : 0.0f, eu, O);
         }
         m = bm;
         c0 += BATCH * SLOTS;
@@ -422,8 +424,9 @@ hipError_t launch_gqa_form(const GqaArgs& a, int parts, hipStream_t s)
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess || chunks == 1)
         return e;
-    // one round trip for every chunk count of the cache (two at 256-value
-    // heads past 64 chunks), with no more slots and loads than that takes
+    // no more slots and loads than one round trip for every chunk takes, up to
+    // 128 chunks (64 at 256-value heads); the 256 chunks of 16384 rows over one
+    // KV head take two (four)
     const dim3 heads(static_cast<unsigned>(a.query_heads));
     if (chunks <= 8)
         hipLaunchKernelGGL((gqa_merge_kernel<HEAD, CHUNK, 1, 8>), heads, dim3(HEAD), 0, s, a);

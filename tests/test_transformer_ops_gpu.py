@@ -183,6 +183,30 @@ def test_grouped_query_attention_forms(hip, fmt, heads, kv_heads, head, context,
     _close(out, t64, 1e-4, "attention vs fp64")
 
 
+# one live chunk of many, a last chunk of one row, and merges of one and more
+# batches, in every head size
+@pytest.mark.parametrize("heads,kv_heads,head,context,position",
+                         [(4, 2, 64, 129, 5), (32, 4, 64, 4096, 100), (2, 1, 64, 16384, 64), (6, 2, 128, 2048, 128),
+                          (8, 1, 128, 16384, 9000), (4, 1, 256, 700, 64), (5, 1, 256, 16384, 3000)])
+def test_grouped_query_attention_ignores_what_the_workspace_held(hip, heads, kv_heads, head, context, position):
+    rng = np.random.default_rng(context + position)
+    q = hip.to_device(rng.standard_normal(heads * head).astype(np.float32))
+    cache = rng.standard_normal((2, context, kv_heads, head)).astype(np.float16)
+    k, v = hip.to_device(cache[0]), hip.to_device(cache[1])
+    p, out = hip.to_device(np.array([position], np.int32)), hip.alloc(4 * heads * head)
+    ws = hip.alloc(native.gqa_workspace_bytes(heads, head, context))
+    outs = []
+    for bits in (0, 0x7fc00000, 0x7f800000, 0xff800000, 0x7f7fffff):   # zeros, NaN, +inf, -inf, the largest value
+        hip.fill_u32(ws.ptr, bits, ws.nbytes // 4)
+        hip.grouped_query_attention(native.GqaArgs(q.ptr, k.ptr, v.ptr, p.ptr, out.ptr, native.F16, heads, kv_heads, head,
+                                                   context, ws.ptr))
+        outs.append(out.readback(np.uint32))
+    assert np.isfinite(outs[0].view(np.float32)).all()
+    assert all(np.array_equal(o, outs[0]) for o in outs[1:])
+    for b in (q, k, v, p, out, ws):
+        b.free()
+
+
 def test_op_rejections(hip):
     buf = hip.alloc(1 << 20)
     p = buf.ptr
