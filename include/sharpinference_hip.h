@@ -231,9 +231,10 @@ typedef struct si_hip_attention {
     const int32_t* position;   /* device scalar: the new token's index = its cache slot */
     void* k_cache;             /* fp16 [kv_heads][capacity][128], 16-byte aligned */
     void* v_cache;             /* fp16 [kv_heads][capacity][128], 16-byte aligned */
-    float* out;                /* [heads * 128] */
-    float* workspace;          /* si_hip_attention_workspace_bytes: chunk partials and the rotary table; any
-                                  contents on entry (each call prepares it); calls that share one workspace
+    float* out;                /* [heads * 128]; where it lies over qkv or a cache it is written after
+                                  everything was read */
+    float* workspace;          /* si_hip_attention_workspace_bytes: chunk partials (and the rotary table of
+                                  a decode step); any contents on entry; calls that share one workspace
                                   must not overlap on the GPU */
     int heads;
     int kv_heads;              /* heads / kv_heads in 1..4 */
@@ -257,7 +258,7 @@ int si_hip_attention_workspace_bytes(int heads, int capacity, uint64_t* bytes);
 int si_hip_attention_decode(si_hip_context* ctx, const si_hip_attention* args);
 
 /* si_hip_attention_decode without a workspace: args->workspace must be
- * NULL, and the chunk partials and rotary table go to a device array of the
+ * NULL, and the chunk partials go to a device array of the
  * library (2 MiB per GPU, held until the process ends), so the call
  * allocates nothing (no hipMalloc, no allocating library routine).  Requests
  * whose workspace (si_hip_attention_workspace_bytes) exceeds 2 MiB, i.e.

@@ -895,6 +895,28 @@ hipError_t launch_combine(const AttentionArgs& a, int limit, int chunks, int chu
     return hipGetLastError();
 }
 
+namespace {
+
+bool meets(const void* a, int64_t abytes, const void* b, int64_t bbytes)
+{
+    const uintptr_t p = reinterpret_cast<uintptr_t>(a), q = reinterpret_cast<uintptr_t>(b);
+    return p < q + static_cast<uintptr_t>(bbytes) && q < p + static_cast<uintptr_t>(abytes);
+}
+
+// A grid of one chunk needs no merge: its workgroups write the output
+// themselves, unless that meets memory another workgroup may still be reading
+// (out == qkv is safe: a workgroup has read its own queries).  Such calls keep
+// the merge, which runs after every read.
+bool writes_directly(const AttentionArgs& a, unsigned chunks)
+{
+    const int64_t out = static_cast<int64_t>(a.heads) * HEAD_DIM * 4;
+    const int64_t kv = static_cast<int64_t>(a.kv_heads) * HEAD_DIM;
+    return chunks == 1 && (a.out == a.qkv || !meets(a.out, out, a.qkv, out + 8 * kv)) &&
+           !meets(a.out, out, a.k_cache, 2 * kv * a.capacity) && !meets(a.out, out, a.v_cache, 2 * kv * a.capacity);
+}
+
+}  // namespace
+
 hipError_t launch_attention(const AttentionArgs& a, hipStream_t s, bool own_table)
 {
     if (a.head_dim != HEAD_DIM || a.kv_heads <= 0 || a.heads % a.kv_heads != 0 || a.max_chunks > MAX_CHUNKS ||
@@ -911,7 +933,7 @@ hipError_t launch_attention(const AttentionArgs& a, hipStream_t s, bool own_tabl
         // slices of 8 values and their rotary partners are whole
         if (bounded && own_table)
             return hipErrorNotSupported;   // bounded grids belong to a step, which has its table
-        float* const direct = fgrid.y == 1 ? a.out : nullptr;
+        float* const direct = writes_directly(a, fgrid.y) ? a.out : nullptr;
         switch (group * 4 + (bounded ? 2 : 0) + (own_table ? 1 : 0)) {
 #define SI_CHUNK(G, B, O)                                                                                         \
     case G * 4 + 2 * B + O:                                                                                       \

@@ -215,6 +215,40 @@ def test_attention_position_outside_cache_yields_nan_and_writes_nothing(hip):
         b.free()
 
 
+# out in the queries, across them, in the keys and values of every KV head and
+# in the cache, in floats from the start of the buffer that holds
+# [qkv | spare | keys | values]; 1024 + 512 floats of qkv
+@pytest.mark.parametrize("capacity,position", [(100, 99), (128, 3), (300, 200)])
+@pytest.mark.parametrize("shift", [0, 32, 128, 900, 1024, 1100, 1280, 1500, 4096 + 64, 4096 + 128 * 130])
+def test_attention_output_over_its_own_operands(hip, capacity, position, shift):
+    """An output that lies in qkv or in a cache is written after everything was
+    read: the same bits as into a buffer of its own."""
+    heads, kv_heads, d = 8, 2, 128
+    rng = np.random.default_rng(capacity + shift)
+    n = (heads + 2 * kv_heads) * d
+    half = kv_heads * capacity * d // 2                       # floats of one fp16 cache
+    host = np.zeros(4096 + 2 * half, np.float32)
+    host[:n] = rng.standard_normal(n)
+    host[4096:] = rng.standard_normal((2, 2 * half)).astype(np.float16).view(np.float32).reshape(-1)
+    buf, out = hip.alloc(host.nbytes), hip.alloc(4 * heads * d)
+    dpos = hip.to_device(np.array([position], np.int32))
+    ws = hip.alloc(native.attention_workspace_bytes(heads, capacity))
+
+    def run(dst):
+        buf.upload(host)
+        hip.attention(native.AttentionArgs(buf.ptr, dpos.ptr, buf.ptr + 4 * 4096, buf.ptr + 4 * (4096 + half), dst, ws.ptr,
+                                           heads, kv_heads, d, 96, capacity, 10000.0, 1.0))
+
+    run(out.ptr)
+    want = out.readback(np.uint32)
+    assert np.isfinite(want.view(np.float32)).all()
+    for _ in range(5):
+        run(buf.ptr + 4 * shift)
+        assert np.array_equal(buf.readback(np.uint32)[shift:shift + heads * d], want)
+    for b in (buf, out, dpos, ws):
+        b.free()
+
+
 def test_argmax_matches_first_index_rule(hip):
     ws = hip.alloc(native.argmax_workspace_bytes())
     out = hip.alloc(4)
