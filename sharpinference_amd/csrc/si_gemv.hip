@@ -990,24 +990,23 @@ int kind_of(const GemvOp& op)
     return nb <= SHORT_MAX_BLOCKS && op.cols <= SHORT_MAX_COLS ? PATH_SHORT : PATH_GENERIC;
 }
 
-// The streaming kernel takes a PATH_GENERIC op that is not pinned to the
-// any-shape kernel.
-bool stream_ok(const GemvOp& op)
+// The streaming kernel takes an op that is not pinned to the any-shape kernel,
+// with weights at an even address; short rows from 128 columns on: one lane
+// decoding a block byte by byte against 16 lanes a row, Q4_K 8000 x 1792 10.9
+// and 5.1 us, 24000 x 256 8.5 and 4.8, Q4_0 16000 x 992 8.6 and 5.3, Q8_0
+// 2048 x 256 2.70 and 2.59; at 64 columns the short-row kernel is ahead (Q4_0
+// 5000 x 64 2.40 and 2.74).  The op alone decides, not the ops beside it in a
+// launch: its result has the same bits in any batch.
+bool streams(const GemvOp& op, int kind)
 {
-    return !op.any_shape && (reinterpret_cast<uintptr_t>(op.w) & 1u) == 0 && op.cols >= 32;
+    return kind != PATH_FAST && !op.any_shape && (reinterpret_cast<uintptr_t>(op.w) & 1u) == 0 &&
+           op.cols >= (kind == PATH_SHORT ? 128 : 32);
 }
 
-// Short rows run there too from 128 columns on, where a launch's ops all do
-// (a launch is not split for it): one lane decoding a block byte by byte
-// against 16 lanes a row, Q4_K 8000 x 1792 10.9 and 5.1 us, 24000 x 256 8.5
-// and 4.8, Q4_0 16000 x 992 8.6 and 5.3, Q8_0 2048 x 256 2.70 and 2.59; at 64
-// columns the short-row kernel is ahead (Q4_0 5000 x 64 2.40 and 2.74).
-bool short_streams(const GemvOp& op) { return stream_ok(op) && op.cols >= 128; }
-
-hipError_t launch_group(const GemvOp* ops, int n, int kind, bool stream, hipStream_t s)
+hipError_t launch_group(const GemvOp* ops, int n, int kind, hipStream_t s)
 {
     const int fmt = ops[0].fmt;
-    if (stream)
+    if (streams(ops[0], kind))
         return launch_gemv_stream(ops, n, s);
     if (kind == PATH_GENERIC || kind == PATH_SHORT) {
         const bool sh = kind == PATH_SHORT;
@@ -1035,22 +1034,19 @@ hipError_t launch_group(const GemvOp* ops, int n, int kind, bool stream, hipStre
 
 }  // namespace
 
-hipError_t launch_gemv_ops(const GemvOp* ops, int count, hipStream_t stream, int* paths)
+hipError_t launch_gemv_ops(const GemvOp* ops, int count, hipStream_t s, int* paths)
 {
     int i = 0;
     while (i < count) {
         const int kind = kind_of(ops[i]);
         if (kind != PATH_FAST && ops[i].in != XF_PLAIN)
             return hipErrorNotSupported;
-        bool streams = kind == PATH_GENERIC && stream_ok(ops[i]);
+        const bool stream = streams(ops[i], kind);
         int n = 1;
         while (i + n < count && n < MAX_SEGS && ops[i + n].fmt == ops[i].fmt && kind_of(ops[i + n]) == kind &&
-               (kind != PATH_FAST || ops[i + n].cols == ops[i].cols) &&
-               (kind != PATH_GENERIC || stream_ok(ops[i + n]) == streams))
+               (kind != PATH_FAST || ops[i + n].cols == ops[i].cols) && streams(ops[i + n], kind) == stream)
             n++;
-        if (kind == PATH_SHORT)
-            streams = std::all_of(ops + i, ops + i + n, short_streams);
-        const hipError_t e = launch_group(ops + i, n, kind, streams, stream);
+        const hipError_t e = launch_group(ops + i, n, kind, s);
         if (e != hipSuccess)
             return e;
         if (paths)

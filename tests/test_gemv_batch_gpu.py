@@ -164,6 +164,58 @@ def test_any_shape_batch_of_short_products(hip):
     B.free()
 
 
+# (rows, columns in 32-column blocks or, for Q4_K, its super-blocks, output,
+# weight offset): short rows on both sides of 128 columns, rows of one to many
+# steps, one row to a ragged 4099 (taller together than the two-rows-a-lane
+# line), one op at an odd address among the others
+UNTABLED = [(33, 2, native.OUT_PLAIN, 0), (50, 8, native.OUT_PLAIN, 0), (1, 33, native.OUT_PLAIN, 2),
+            (4099, 130, native.OUT_PLAIN, 0), (40, 35, native.OUT_SWIGLU_ROWS, 0), (9, 33, native.OUT_PLAIN, 1),
+            (17, 375, native.OUT_TANH, 0), (300, 34, native.OUT_RELU_SQUARE, 0), (5, 3, native.OUT_SIGMOID, 0),
+            (2100, 31, native.OUT_PLAIN, 0)]
+
+
+@pytest.mark.parametrize("fmt", FORMATS + [native.F16, native.F32])
+def test_untabled_ops_of_a_batch(hip, fmt):
+    """Ops outside the tiled kernel's column table, of different heights,
+    widths, outputs and residuals, in one call: each within the GEMV gate
+    (doubled through relu^2, SwiGLU and tanh) and bit-identical to the op
+    launched alone."""
+    B = Bufs(hip)
+    ops, ref, ys, sizes = [], [], [], []
+    for i, (rows, nb, out, offset) in enumerate(UNTABLED):
+        cols = nb * 32 if fmt in (native.Q8_0, native.Q4_0) else 256 * max(1, nb // 8) if fmt == native.Q4_K else nb * 32 - 7
+        wrows = 2 * rows if out == native.OUT_SWIGLU_ROWS else rows
+        if fmt in FORMATS:
+            w = orc.gen_quant(fmt, 500 + i, wrows, cols)
+            wd = orc.dequant(fmt, w, wrows, cols)
+        else:
+            wd = orc.gen_normal_f32(500 + i, wrows * cols, 0.0, 0.02)
+            wd = wd.astype(np.float16) if fmt == native.F16 else wd
+            w = wd.view(np.uint8)
+        x, r = orc.gen_normal_f32(600 + i, cols), orc.gen_normal_f32(700 + i, rows)
+        dw = hip.alloc(w.nbytes + offset)
+        B.items.append(dw)
+        dw.upload(w, offset=offset)
+        dx, dr, dy = B.up(x), B.up(r), B.out(rows)
+        plain = out == native.OUT_PLAIN
+        ops.append(native.gemv_op(fmt, dw.ptr + offset, dx.ptr, dy.ptr, rows, cols, output=out, residual=dr.ptr if plain else 0))
+        t = wd.reshape(wrows, cols).astype(np.float64) @ x.astype(np.float64)
+        ref.append({native.OUT_PLAIN: lambda: t + r, native.OUT_TANH: lambda: np.tanh(t),
+                    native.OUT_SIGMOID: lambda: 1 / (1 + np.exp(-t)), native.OUT_RELU_SQUARE: lambda: np.maximum(t, 0) ** 2,
+                    native.OUT_SWIGLU_ROWS: lambda: t[:rows] / (1 + np.exp(-t[:rows])) * t[rows:]}[out]())
+        ys.append(dy)
+        sizes.append(rows)
+    paths = hip.gemv_batch(ops)
+    together = [y.readback(np.float32, n) for y, n in zip(ys, sizes)]
+    for i, op in enumerate(ops):
+        close(together[i], ref[i], 2e-3, 2e-5, f"op {i}")
+        hip.fill_u32(ys[i].ptr, 0x7fc00000, sizes[i])
+        assert hip.gemv_batch([op]) == [paths[i]]
+        alone = ys[i].readback(np.float32, sizes[i])
+        assert np.array_equal(together[i].view(np.uint32), alone.view(np.uint32)), f"op {i}: other bits beside its neighbours"
+    B.free()
+
+
 def test_batch_rejects_dependences_and_bad_ops(hip):
     fmt, rows, cols = native.Q8_0, 64, 1024
     w = orc.gen_quant(fmt, 1, rows, cols)
