@@ -1008,13 +1008,15 @@ __device__ __forceinline__ void decode_staged(const uint8_t* row, int b, int g, 
         const uint8_t* blk = row + ((18 * b) & 15);
         const float d = half_bits(lds_u16(blk));
         const uint32_t q = lds_u16(blk + 2 + 4 * g) | (lds_u16(blk + 4 + 4 * g) << 16);   // qs[4g..4g+3]
-        float nl[4], nh[4];
-        bytes_to_float(q & 0x0F0F0F0Fu, nl);          // one nibble per byte
-        bytes_to_float((q >> 4) & 0x0F0F0F0Fu, nh);
+        // n ^ 8 is n - 8 as a signed nibble; at the top of a byte it reads as
+        // 16 (n - 8), the 16 taken from the scale (both exact, and an infinite
+        // scale keeps the decode's signs: fma(d, n, -8 d) would be NaN)
+        const uint32_t t = q ^ 0x88888888u, lo = (t << 4) & 0xF0F0F0F0u, hi = t & 0xF0F0F0F0u;
+        const float d16 = d * 0.0625f;
 #pragma unroll
-        for (int e = 0; e < 4; e++) {   // d (n - 8): every term is exact in FP32
-            w[e] = fmaf(d, nl[e], -8.0f * d);       // element 4g+e
-            w[4 + e] = fmaf(d, nh[e], -8.0f * d);   // element 16+4g+e
+        for (int e = 0; e < 4; e++) {
+            w[e] = d16 * static_cast<float>(static_cast<int8_t>(lo >> (8 * e)));       // element 4g+e
+            w[4 + e] = d16 * static_cast<float>(static_cast<int8_t>(hi >> (8 * e)));   // element 16+4g+e
         }
     } else {   // Q4_K sub-block j of the super-block (j is the same for the whole wave)
         const int j = b & 7;

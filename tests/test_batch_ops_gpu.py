@@ -18,6 +18,7 @@ import pytest
 
 import oracle as orc
 from sharpinference_amd import native
+from tests import blocks
 from tests.test_gemv_gpu import assert_gemv_close
 
 pytestmark = pytest.mark.gpu
@@ -160,6 +161,35 @@ def test_batch_matvec(hip, fmt, rows, cols, batch, valid):
     for t in range(valid):
         assert_gemv_close(got[t], orc.gemv_f64(fmt, w, x[t], rows, cols), f"format {fmt} row {t}")
     assert np.all(got[valid:] == SENTINEL)
+    for b in (dw, dx, ctl, dy):
+        b.free()
+
+
+@pytest.mark.parametrize("cols", [256, 288, 1280])
+def test_batch_matvec_infinite_q4_0_scale(hip, cols):
+    """A block whose fp16 scale is infinite decodes to +-inf by the sign of n - 8
+    (NaN for n = 8) on the LDS-ring form (columns % 256 == 0) and the other
+    alike."""
+    rng = np.random.default_rng(cols)
+    nb = cols // 32
+    nib = rng.integers(0, 16, (8, nb, 32))
+    d = rng.uniform(0.001, 0.01, (8, nb))
+    for row, (scale, values) in enumerate([(np.inf, range(9, 16)), (np.inf, range(0, 8)), (-np.inf, range(9, 16)),
+                                           (-np.inf, range(0, 8)), (np.inf, [8] + 31 * [12]), (np.inf, 16 * [3] + 16 * [12]),
+                                           (np.nan, range(16))]):   # the last row stays finite
+        d[row, nb // 2] = scale
+        nib[row, nb // 2] = np.resize(list(values), 32)
+    w = blocks.q4_0(d.reshape(-1), nib)
+    x = (0.1 + np.abs(rng.standard_normal((16, cols)))).astype(np.float32)
+    dw, dx, ctl, dy = hip.to_device(w), hip.to_device(x), _control(hip, 100, 16), _filled(hip, (16, 8))
+    hip.batch_matvec(native.Q4_0, dw.ptr, dx.ptr, ctl.ptr, dy.ptr, 16, 8, cols)
+    got = dy.readback(np.float32).reshape(16, 8)
+    with np.errstate(invalid="ignore"):
+        want = x.astype(np.float64) @ orc.dequant(native.Q4_0, w, 8, cols).reshape(8, cols).astype(np.float64).T
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    assert np.array_equal(got[np.isinf(got)], want[np.isinf(want)].astype(np.float32))
+    assert list(np.isinf(want[0])) == [True] * 4 + [False] * 4 and list(np.isnan(want[0])) == [False] * 4 + [True] * 3 + [False]
+    assert_gemv_close(got[:, 7], want[:, 7], "finite row")
     for b in (dw, dx, ctl, dy):
         b.free()
 
