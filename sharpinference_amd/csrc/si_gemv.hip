@@ -991,16 +991,20 @@ int kind_of(const GemvOp& op)
 }
 
 // The streaming kernel takes an op that is not pinned to the any-shape kernel,
-// with weights at an even address; short rows from 128 columns on: one lane
-// decoding a block byte by byte against 16 lanes a row, Q4_K 8000 x 1792 10.9
-// and 5.1 us, 24000 x 256 8.5 and 4.8, Q4_0 16000 x 992 8.6 and 5.3, Q8_0
-// 2048 x 256 2.70 and 2.59; at 64 columns the short-row kernel is ahead (Q4_0
-// 5000 x 64 2.40 and 2.74).  The op alone decides, not the ops beside it in a
-// launch: its result has the same bits in any batch.
+// with weights at an even address; of the short rows those of more than 256
+// columns and all of Q4_K: one lane decoding a block byte by byte against 16
+// lanes a row, Q4_K 24000 x 256 8.5 and 4.8 us, 8000 x 1792 10.9 and 5.1; Q8_0
+// 2048 x 512 3.17 and 2.92, 16384 x 992 9.6 and 6.9, Q4_0 8.5 and 4.6.  Up to 256
+// columns neither leads by more than launches vary (Q8_0 2048 x 256 2.75 and
+// 2.57, 16384 x 256 3.67 and 3.79, Q4_0 16384 x 128 2.97 and 3.36, 5000 x 64 2.40
+// and 2.74), and the RWKV-7 LoRA outputs (64 to 256 columns) stay one launch:
+// one of four such ops takes 3.1 us, split in three 7.5.  The op alone decides,
+// not the ops beside it: its result has the same bits in any batch.
 bool streams(const GemvOp& op, int kind)
 {
-    return kind != PATH_FAST && !op.any_shape && (reinterpret_cast<uintptr_t>(op.w) & 1u) == 0 &&
-           op.cols >= (kind == PATH_SHORT ? 128 : 32);
+    if (kind == PATH_FAST || op.any_shape || (reinterpret_cast<uintptr_t>(op.w) & 1u) != 0)
+        return false;
+    return kind == PATH_SHORT ? op.fmt == FMT_Q4_K || op.cols > 256 : op.cols >= 32;
 }
 
 hipError_t launch_group(const GemvOp* ops, int n, int kind, hipStream_t s)

@@ -165,12 +165,12 @@ def test_any_shape_batch_of_short_products(hip):
 
 
 # (rows, columns in 32-column blocks or, for Q4_K, its super-blocks, output,
-# weight offset): short rows on both sides of 128 columns, rows of one to many
+# weight offset): short rows on both sides of 256 columns, rows of one to many
 # steps, one row to a ragged 4099 (taller together than the two-rows-a-lane
 # line), one op at an odd address among the others
 UNTABLED = [(33, 2, native.OUT_PLAIN, 0), (50, 8, native.OUT_PLAIN, 0), (1, 33, native.OUT_PLAIN, 2),
             (4099, 130, native.OUT_PLAIN, 0), (40, 35, native.OUT_SWIGLU_ROWS, 0), (9, 33, native.OUT_PLAIN, 1),
-            (17, 375, native.OUT_TANH, 0), (300, 34, native.OUT_RELU_SQUARE, 0), (5, 3, native.OUT_SIGMOID, 0),
+            (17, 375, native.OUT_TANH, 0), (300, 34, native.OUT_RELU_SQUARE, 0), (5, 9, native.OUT_SIGMOID, 0),
             (2100, 31, native.OUT_PLAIN, 0)]
 
 

@@ -434,7 +434,7 @@ STREAM = [(native.Q8_0, 1, 1056), (native.Q8_0, 4099, 2080), (native.Q8_0, 17, 4
           (native.Q4_K, 1, 2304), (native.Q4_K, 5001, 11008), (native.Q4_K, 4097, 2304), (native.Q4_K, 16, 8448),
           (native.F16, 3, 33), (native.F16, 300, 777), (native.F16, 5, 11007), (native.F16, 1000, 256),
           (native.F32, 2, 63), (native.F32, 65, 4097), (native.F32, 9, 512),
-          # short rows from 128 columns on
+          # short rows (Q8_0 and Q4_0 up to 256 columns on the short-row kernel)
           (native.Q8_0, 5, 128), (native.Q8_0, 16001, 512), (native.Q4_0, 33, 992), (native.Q4_K, 8001, 1792),
           (native.Q4_K, 17, 256)]
 STREAM_NAMES = {**NAMES, native.F16: "f16", native.F32: "f32"}
