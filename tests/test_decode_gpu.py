@@ -249,6 +249,30 @@ def test_attention_output_over_its_own_operands(hip, capacity, position, shift):
         b.free()
 
 
+# positions that leave most, or all but one, of the merge's chunks unwritten
+@pytest.mark.parametrize("rotary", [96, 40])
+@pytest.mark.parametrize("capacity,position", [(129, 5), (256, 255), (1024, 128), (1100, 900), (4096, 0), (4200, 1500),
+                                               (8192, 127), (16384, 130), (16384, 9000)])
+def test_attention_ignores_what_the_workspace_held(hip, capacity, position, rotary):
+    heads, kv_heads, d = 6, 2, 128
+    rng = np.random.default_rng(capacity + position)
+    dq = hip.to_device(rng.standard_normal((heads + 2 * kv_heads) * d).astype(np.float32))
+    cache = rng.standard_normal((2, kv_heads, capacity, d)).astype(np.float16)
+    dk, dv = hip.to_device(cache[0]), hip.to_device(cache[1])
+    dpos, dout = hip.to_device(np.array([position], np.int32)), hip.alloc(4 * heads * d)
+    ws = hip.alloc(native.attention_workspace_bytes(heads, capacity))
+    outs = []
+    for bits in (0, 0x7fc00000, 0x7f800000, 0xff800000, 0x7f7fffff):   # zeros, NaN, +inf, -inf, the largest value
+        hip.fill_u32(ws.ptr, bits, ws.nbytes // 4)
+        hip.attention(native.AttentionArgs(dq.ptr, dpos.ptr, dk.ptr, dv.ptr, dout.ptr, ws.ptr, heads, kv_heads, d, rotary,
+                                           capacity, 10000.0, 1.0))
+        outs.append(dout.readback(np.uint32))
+    assert np.isfinite(outs[0].view(np.float32)).all()
+    assert all(np.array_equal(o, outs[0]) for o in outs[1:])
+    for b in (dq, dk, dv, dpos, dout, ws):
+        b.free()
+
+
 def test_argmax_matches_first_index_rule(hip):
     ws = hip.alloc(native.argmax_workspace_bytes())
     out = hip.alloc(4)

@@ -127,7 +127,8 @@ def test_layernorm_and_relu_square(hip, fmt, rows, cols):
 @pytest.mark.parametrize("cols", [3072, 256])
 def test_swiglu_rows(hip, fmt, cols):
     """W = [gate rows; up rows]: y_r = silu(g_r) * u_r, on the tiled kernel
-    (cols 3072, RMSNorm staged) and the any-shape kernel (cols 256)."""
+    (cols 3072, RMSNorm staged) and, at 256 columns, the short-row (Q8_0,
+    Q4_0) or the streaming kernel (Q4_K)."""
     F = 1536
     w = orc.gen_quant(fmt, 11, 2 * F, cols)
     x = orc.gen_normal_f32(12, cols, 0.0, 1.0)

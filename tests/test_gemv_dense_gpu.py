@@ -69,7 +69,7 @@ def test_dense_any_shape_path_matches_oracle(hip, fmt, rows, cols):
     w = dense(fmt, rows, cols, 20 + rows)
     x = orc.gen_normal_f32(21 + cols, cols)
     # a 2-byte offset leaves the rows without dword alignment: the 3072-column
-    # shapes take the any-shape kernel too
+    # shapes take the streaming kernel too (up to 32 columns the short-row one)
     y, path = run_gemv(hip, fmt, w, x, rows, cols, w_offset=2 if cols == 3072 else 0)
     assert path == (native.PATH_SHORT if cols <= 32 else native.PATH_GENERIC)
     assert_gemv_close(y, orc.gemv_f64(fmt, w, x, rows, cols))

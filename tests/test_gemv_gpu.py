@@ -91,8 +91,9 @@ GENERIC = [(native.Q8_0, 513, 4160), (native.Q4_0, 65, 96), (native.Q4_K, 9, 230
 def test_any_shape_path_matches_oracle(hip, fmt, rows, cols):
     w = orc.gen_quant(fmt, 5 + rows, rows, cols)
     x = orc.gen_normal_f32(6 + cols, cols)
-    # a 2-byte offset leaves W without dword alignment, which routes 3072
-    # columns to the any-shape kernel as well
+    # a 2-byte offset leaves W without dword alignment, which takes 3072
+    # columns off the tiled kernel (these run the streaming kernel or, up to
+    # 256 columns of Q8_0 and Q4_0, the short-row one)
     y, path = run_gemv(hip, fmt, w, x, rows, cols, w_offset=2 if cols == 3072 else 0)
     short = cols // native.BLOCK_ELEMS[fmt] <= 32 and cols <= 2048
     assert path == (native.PATH_SHORT if short else native.PATH_GENERIC)
@@ -540,6 +541,37 @@ def test_streaming_dense_rows_sum_in_short_chains(hip, fmt, cols):
         t = orc.gemv_f64(fmt, w, x, rows, cols)
         squares.append(np.sum((y - t) ** 2) / np.sum(t * t))
     assert np.sqrt(np.mean(squares)) <= 1.47 * 2.0 ** -24
+
+
+# Weights at an odd address: the byte-by-byte kernels (one wave per row; one
+# lane per block of a short row) of every format.
+ODD_ADDRESS = [(f, *c) for f in (native.Q8_0, native.Q4_0) for c in [(33, 64), (300, 992), (65, 1056), (9, 3072)]] + \
+              [(native.Q4_K, *c) for c in [(5, 256), (100, 1792), (65, 2304), (9, 3072)]] + \
+              [(f, *c) for f in (native.F16, native.F32) for c in [(7, 17), (5, 32), (300, 777), (9, 3072)]]
+
+
+@pytest.mark.parametrize("fmt,rows,cols", ODD_ADDRESS, ids=[f"{STREAM_NAMES[f]}-{r}x{c}" for f, r, c in ODD_ADDRESS])
+def test_weights_at_odd_addresses_match_oracle(hip, fmt, rows, cols):
+    """A product with a residual, and SwiGLU rows beside a second product in
+    one call, each with the bits it has alone."""
+    w = orc.gen_quant(fmt, 15 + rows, 2 * rows, cols) if fmt in NAMES else _dense(fmt, 2 * rows, cols, 15 + rows)
+    x, r = orc.gen_normal_f32(16 + cols, cols), orc.gen_normal_f32(17 + cols, rows)
+    t = orc.gemv_f64(fmt, w, x, 2 * rows, cols)
+    short = cols // native.BLOCK_ELEMS.get(fmt, 1) <= 32 and cols <= 2048
+    path = native.PATH_SHORT if short else native.PATH_GENERIC
+    dw = hip.alloc(w.nbytes + 1)
+    dw.upload(w, offset=1)
+    dx, dr, dy, dz = hip.to_device(x), hip.to_device(r), hip.alloc(4 * rows), hip.alloc(4 * rows)
+    assert hip.gemv(fmt, dw.ptr + 1, dx.ptr, dy.ptr, rows, cols, residual=dr.ptr) == path
+    y = dy.readback(np.float32, rows)
+    assert_gemv_close(y, t[:rows] + r)
+    ops = [native.gemv_op(fmt, dw.ptr + 1, dx.ptr, dz.ptr, rows, cols, output=native.OUT_SWIGLU_ROWS),
+           native.gemv_op(fmt, dw.ptr + 1, dx.ptr, dy.ptr, rows, cols, residual=dr.ptr)]
+    assert hip.gemv_batch(ops) == [path, path]
+    assert np.array_equal(dy.readback(np.float32, rows), y)
+    assert_gemv_close(dz.readback(np.float32, rows), t[:rows] / (1 + np.exp(-t[:rows])) * t[rows:], "swiglu rows")
+    for b in (dw, dx, dr, dy, dz):
+        b.free()
 
 
 # ---- plans of a few kernels ---------------------------------------------------------------
