@@ -19,31 +19,12 @@
 // 45.0 (4.5 TB/s), 34.4 -> 31.6.  The block formats keep the LDS ring: here they
 // took 8.6 to 9.5 us for 3072 x 3072 against 8.0 to 8.6.
 #include "si_batch.hpp"
-#include "si_internal.hpp"
-
-#include <hip/hip_fp16.h>
+#include "si_prefill_units.hpp"
 
 namespace si {
 namespace {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
 constexpr int MV_WAVES = 8;
-
-__device__ __forceinline__ float half_bits(uint32_t h)
-{
-    return __half2float(__ushort_as_half(static_cast<unsigned short>(h & 0xffffu)));
-}
-
-// Keeps a lane offset 32-bit beside a scalar base, and a masked word's zero
-// bits hidden (one v_cvt_f32_ubyteN per byte).
-__device__ __forceinline__ uint32_t opaque(uint32_t v)
-{
-    asm("" : "+v"(v));
-    return v;
-}
 
 // Part q (0..3) of a row's 64-column step: columns 8q .. 8q + 7 of both
 // 32-column blocks, 4 (F16) or 8 (F32) words of each.

@@ -1,6 +1,7 @@
-// W decode shared by the prefill products (si_prefill.hip,
-// si_prefill_skinny.hip): the raw words of 16 values of a weight row and their
-// exact values rounded to bf16.
+// Parts of the prefill products: the W decode of si_prefill.hip and
+// si_prefill_skinny.hip (the raw words of 16 values of a weight row and their
+// exact values rounded to bf16), and the vector types and word helpers that
+// si_batch_matvec.hip uses too.
 #pragma once
 
 #include "si_internal.hpp"
@@ -18,9 +19,9 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));   // 16 raw bytes
 
 // Raw words of one item of 16 values (half a 32-value block of one W row),
-// loaded steps ahead of their decode.  The loads are plain word loads and
-// every bit extraction happens at decode time, so a word in flight is never
-// touched before its decode.  An F32 item is 16 words, every other format's
+// loaded steps ahead of their decode.  Loads of up to 16 bytes bring whole
+// words and every bit extraction happens at decode time, so a word in flight is
+// never touched before its decode.  An F32 item is 16 words, every other format's
 // at most 8.
 template <int FMT>
 struct RawW {
