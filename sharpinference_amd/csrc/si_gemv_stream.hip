@@ -14,9 +14,10 @@
 // unit (F16 / F32) are taken two per lane by the first slice.
 //
 // Bound: the decode and FP32 products of the 4-bit formats (Q4_K about 2.7
-// vector instructions a weight), HBM for the others.  The generic kernel reads
+// vector instructions a weight, their units busy for 0.66 of 20000 x 5120), the
+// address unit (busy 0.7) on the way to HBM for the others.  The generic kernel reads
 // byte by byte, a wave a row.  Against it, weights from HBM: Q4_K 5001 x 11008
-// 43.5 -> 12.8 us (2.4 TB/s), Q8_0 16000 x 5120 51 -> 18 us (4.8 TB/s), F16
+// 43.5 -> 12.1 us (2.6 TB/s), Q8_0 16000 x 5120 51 -> 18 us (4.8 TB/s), F16
 // 24000 x 3500 86 -> 32 us (5.2 TB/s), F32 64 x 14000 66 -> 9 us.  With 8
 // waves a workgroup the grids' last wave cost more (F16 41 us).
 #include "si_gemv_units.hpp"
@@ -44,7 +45,7 @@ __device__ __forceinline__ void ld4_a2(const uint8_t* p, uint32_t* v)
 // times 2^-24, or 1024 + n with the exponent's bits set), which v_fma_mix_f32
 // multiplies in FP32.  That takes no more time than one conversion a weight
 // and the sums did (Q4_K 8000 x 1792 6.85 -> 6.25 us, 5001 x 11008 12.3 ->
-// 12.8, Q4_0 16000 x 992 5.6 -> 5.5).
+// 12.1, Q4_0 16000 x 992 5.6 -> 5.5).
 template <int FMT>
 struct SUnit;
 
@@ -353,9 +354,13 @@ __global__ __launch_bounds__(64 * STREAM_WAVES) void gemv_stream_kernel(Segs<NS>
 // Waves per row (ks): as many as give each lane at most one unit, up to 4.
 // Rows per lane (RL): two rows of the block formats per staged x value where
 // the grid still gives each CU two workgroups (Q8_0 24000 x 1056 13.4 us with
-// one, 10.2 with two; 100 x 12000 4.6 and 6.3 the other way); four measured
-// no faster, and F16 / F32 rows stream best alone (F16 5001 x 11007 22 us, 27
-// with two).
+// one, 10.2 with two; 100 x 12000 4.6 and 6.3 the other way).  The 4-bit formats'
+// longer decode is shared worse by two or three waves a SIMD, so theirs lies at
+// three (Q4_0) and four (Q4_K): 5001 x 11008, 626 workgroups of two rows, two calls
+// of Q4_K 17.8 us with one row and 20.5 with two, Q4_0 19.5 and 20.7; Q4_K 20000 x
+// 5120, 2500, 18.0 and 17.5; Q4_0 16000 x 992, 1000, 5.8 and 5.5.  Four rows
+// measured no faster, and F16 / F32 rows stream best alone (F16 5001 x 11007 22
+// us, 27 with two).
 template <int FMT, int RL>
 hipError_t launch_stream_rows(const GemvOp* ops, int n, int ks, hipStream_t s)
 {
@@ -384,7 +389,7 @@ hipError_t launch_stream(const GemvOp* ops, int n, hipStream_t s)
     while (ks < STREAM_WAVES && 16 * ks < units)
         ks *= 2;
     if constexpr (is_block_quant(FMT)) {
-        if (rows / (STREAM_WAVES / ks * 8) >= 512)
+        if (rows / (STREAM_WAVES / ks * 8) >= (FMT == FMT_Q8_0 ? 512 : FMT == FMT_Q4_0 ? 768 : 1024))
             return launch_stream_rows<FMT, 2>(ops, n, ks, s);
     }
     return launch_stream_rows<FMT, 1>(ops, n, ks, s);

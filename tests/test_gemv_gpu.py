@@ -428,11 +428,12 @@ def _dense(fmt, rows, cols, seed):
 
 
 # one to many steps of the slices, one row to a ragged last workgroup, one and
-# two rows per lane (>= 4096 rows), odd block counts (rows at 2-byte
-# addresses), dense columns past the last 32
+# two rows per lane (from 4096 rows, Q4_0 6144, Q4_K 8192), odd block counts
+# (rows at 2-byte addresses), dense columns past the last 32
 STREAM = [(native.Q8_0, 1, 1056), (native.Q8_0, 4099, 2080), (native.Q8_0, 17, 4160), (native.Q8_0, 9001, 1088),
           (native.Q4_0, 5, 1056), (native.Q4_0, 4096, 2112), (native.Q4_0, 33, 12000), (native.Q4_0, 8200, 1120),
           (native.Q4_K, 1, 2304), (native.Q4_K, 5001, 11008), (native.Q4_K, 4097, 2304), (native.Q4_K, 16, 8448),
+          (native.Q4_K, 8200, 2304),
           (native.F16, 3, 33), (native.F16, 300, 777), (native.F16, 5, 11007), (native.F16, 1000, 256),
           (native.F32, 2, 63), (native.F32, 65, 4097), (native.F32, 9, 512),
           # short rows (Q8_0 and Q4_0 up to 256 columns on the short-row kernel)
@@ -504,7 +505,8 @@ def _zero_mean_4bit(fmt, rows, cols, seed):
 
 
 MEANS = [(native.Q4_0, 300, 992), (native.Q4_0, 301, 256), (native.Q4_0, 300, 12000), (native.Q4_0, 4100, 2112),
-         (native.Q4_K, 300, 1792), (native.Q4_K, 300, 11008), (native.Q4_K, 4100, 2304)]
+         (native.Q4_0, 6200, 2112), (native.Q4_K, 300, 1792), (native.Q4_K, 300, 11008), (native.Q4_K, 4100, 2304),
+         (native.Q4_K, 8200, 2304)]
 
 
 @pytest.mark.parametrize("fmt,rows,cols", MEANS, ids=[f"{NAMES[f]}-{r}x{c}" for f, r, c in MEANS])
