@@ -412,8 +412,8 @@ struct QUnit<FMT_F32> {
 // Device copy of one GemvOp.  A launch carries up to MAX_SEGS of them by
 // value.  The tiled kernel runs a 1D grid of exactly the ops' workgroups
 // (op i from workgroup first[i]; a workgroup finds its op with a uniform
-// scan of the kernel arguments); the short-row and any-shape kernels run a
-// 2D grid, grid row i being op i (as wide as the largest op needs), whose
+// scan of the kernel arguments); the streaming, short-row and any-shape kernels
+// run a 2D grid, grid row i being op i (as wide as the largest op needs), whose
 // workgroups past their op's rows leave before any load or barrier.
 struct Seg {
     const uint8_t* w;
@@ -431,7 +431,7 @@ struct Seg {
     int in;                 // XformKind
     int out;                // OutKind
     int copy_n;
-    int blocks;             // blocks per row (generic kernel)
+    int blocks;             // blocks per row (all but the tiled kernel)
     float eps;
 };
 // A launch of one op carries a one-entry table, so its kernel reads its

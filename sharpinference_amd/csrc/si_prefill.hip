@@ -829,30 +829,31 @@ inline int prefill_splits(int64_t tiles, int64_t steps, int cus, int min_steps)
 //       300 x 3072, 400 (70)      10.2 25.1 |  9.6 22.8 |  9.7 21.8 |  9.5 19.5 | 12.0 25.8
 //     (tiles in brackets); past the line, Q8_0 3072 x 3072 at 400 tokens (672)
 //     35.0 and 27.1, 3072 x 8192 at 200 (384) 57.8 and 33.9, 16384 x 3072 at 100
-//     (1024) 53.5 and 45.3.  The figures of the choices below were taken against
-//     each other with word-wide W loads (the wide loads took all of them
-//     further: Q4_K at 2048 tokens 157.8 -> 109.6, 81.9 -> 56.1, 318 -> 234 and
-//     222 -> 130 us for the four projections, F16 212 -> 94, 108 -> 48, 420 ->
-//     218, 269 -> 117);
+//     (1024) 53.5 and 45.3;
 //   * grids of more than 256 workgroups of 256 tokens x 64 rows: the
 //     warp-specialised kernel with 256 x 128 tiles (64 x 128 consumer wave
-//     tiles; gate_up 76 -> 67 us);
+//     tiles);
 //   * with a split buffer, K split over about one workgroup per CU of the
 //     same 256 x 128 tiles (at least 16 steps a split) when the 256 x 64
-//     grid has 128..256 workgroups or K >= 4096: qkv 42.0 -> 37.2 us (3
-//     splits), down 65.5 -> 50.0 us (5 splits); o_proj (3072 columns, 96
-//     workgroups of 256 x 64) stays on the 16 x 16 form (26.4 against 28.2);
+//     grid has 128..256 workgroups or K >= 4096;
 //   * 256 tokens x 64 rows (64 x 64 wave tiles, each fragment used twice)
 //     when that grid has at least 128 workgroups: up to one per
 //     CU two step groups of 4 waves with compact tiles (160 KiB, two waves
 //     per SIMD) when they divide the steps, else the padded tile (84 KiB);
 //   * otherwise, when K is a multiple of 256 and 96-row x 64-token tiles
 //     give 128..256 workgroups, the 16 x 16 block form with that tile, 128
-//     columns per step and the steps split between two groups of 4 waves
-//     (o_proj 28.4 -> 25.7 us, down 72.4 -> 61.0 us at 512 tokens);
+//     columns per step and the steps split between two groups of 4 waves;
 //   * otherwise 128 tokens x 64 rows with the steps split between two
 //     groups of 4 waves when they divide evenly (two waves per SIMD
 //     overlap their phases).
+// The last five at 512 tokens, Q4_0, us, * the rule's (four weights in turn):
+//                   whole K   split   256 x 64   16 x 16   128 x 64
+//   5120 x 3072      52.3     31.6*     36.0       41.0       44.6
+//   3072 x 3072      51.5     27.7      35.1       21.6*      23.5
+//   16384 x 3072     54.1*     -        71.2      120.0       89.3
+//   3072 x 8192     128.3     39.9*     82.1       48.1       55.7
+// The other formats choose alike but at 3072 x 3072, where 128 x 64 and 16 x 16
+// take 26.2 and 27.3 for Q8_0, 22.6 and 22.9 for Q4_K, 26.5 and 32.0 for F32.
 template <int FMT>
 hipError_t launch_prefill_fmt(const void* w, const void* x, float* y, int64_t m, int64_t n, int64_t k, hipStream_t s,
                               void* split)

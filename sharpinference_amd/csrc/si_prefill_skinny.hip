@@ -19,8 +19,9 @@
 // ahead measured no faster than two).
 //
 // Bound: the serial chain of a wave's steps (load, exchange, decode, two
-// products per tile), its LDS and its address work together, on two waves a
-// SIMD.  The four projections of a 3072-wide layer (qkv, o, gate/up, down),
+// products per tile) on two waves a SIMD: half of it is waiting, and no unit is
+// busy for more than 0.6 of the time (address unit 0.3 to 0.6, VALU 0.14 to
+// 0.27, matrix cores 0.05 to 0.10).  The four projections of a 3072-wide layer (qkv, o, gate/up, down),
 // Q8_0 at 33 tokens: 33.6 + 33.5 + 48.4 + 37.9 us with the LDS-tiled kernels,
 // 11.8 + 8.5 + 27.8 + 21.3 us here (161 -> 76 us in one plan); 3072 x 3072 Q4_K at 1 token 29.9 -> 5.6 us,
 // F16 300 x 3072 at 16 51.6 -> 5.0 us.

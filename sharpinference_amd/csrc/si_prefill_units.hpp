@@ -87,7 +87,8 @@ __device__ __forceinline__ uint32_t item_qoff(uint32_t row_off, int bo, int h)
 // Item h of a block, with the widest loads the layout allows (one load
 // instruction costs the address unit about a cycle per four lanes of a row
 // whatever its width: loaded word by word, Q4_K items took twice the
-// matrix-core time of a step) and no vector address arithmetic:
+// matrix-core time of a step; the four projections of a 3072-wide layer at 2048
+// tokens 794 -> 551 us) and no vector address arithmetic:
 //   Q4_0 {fp16 d; u8 qs[16]}: d and bytes 8h..8h+7 (elements 8h..8h+7 in the
 //        low nibbles, 16+8h..16+8h+7 in the high nibbles);
 //   Q8_0 {fp16 d; int8 q[32]}: d and q[16h..16h+15];
